@@ -1,0 +1,104 @@
+// Choice and launch of the W8A8 GEMM's smaller tiles (gemm_tile.h).
+#include "gemm_tile.h"
+
+namespace xgen {
+
+namespace {
+
+// The tiles, smallest first: (waves x, waves y, fragments x, fragments y, pair slots).
+// Slots: as many as keep two workgroups of the small tiles on a CU, and the LDS
+// limit for the large ones (four slots of 128 x 192 measured as three).
+#define XGEN_GEMM_TILES(X) \
+  X(1, 2, 1, 1, 4) /*  32 x  64 */ \
+  X(1, 4, 1, 1, 4) /*  32 x 128 */ \
+  X(2, 2, 1, 1, 4) /*  64 x  64 */ \
+  X(2, 2, 1, 2, 3) /*  64 x 128 */ \
+  X(2, 2, 2, 2, 4) /* 128 x 128 */ \
+  X(2, 2, 2, 3, 3) /* 128 x 192 */ \
+  X(2, 2, 4, 2, 3) /* 256 x 128 */ \
+  X(2, 2, 4, 3, 2) /* 256 x 192 */
+
+constexpr int kTiles = 8;
+struct TileSize {
+  int m, n;
+};
+#define XGEN_TILE_SIZE(WM, WN, FM, FN, S) {TileCfg<WM, WN, FM, FN, S>::kM, TileCfg<WM, WN, FM, FN, S>::kN},
+constexpr TileSize kTileSizes[kTiles + 1] = {XGEN_GEMM_TILES(XGEN_TILE_SIZE){kTileM, kTileN}};
+
+// What a call costs on a tile, in us: start + rounds * (pairs * per_pair + per_tile),
+// rounds = tiles per CU rounded up, pairs = 128-byte steps of K.  Fitted to the times of
+// every tile on 171 shapes per kind (M 2 to 15,624; N x K from 1,024 x 1,024 to
+// 18,432 x 3,072 and 5,376 x 14,336; real-valued operands, so at the clock that the
+// power limit leaves); the choice by these sums is within 0.6% (FP8), 0.5% (INT8) and
+// 0.3% (exact) of the best tile on the average over them, and 10% at worst.  Last row:
+// the 256 x 256 kernel, whose epilogue runs under the next tile.
+struct TileCost {
+  float per_pair, per_tile, start;
+};
+constexpr TileCost kTileCosts[3][kTiles + 1] = {
+    // INT8
+    {{0.152f, 0.0f, 3.7f}, {0.208f, 1.0f, 2.7f}, {0.201f, 0.4f, 3.2f}, {0.286f, 1.5f, 2.4f}, {0.414f, 5.4f, 0.0f},
+     {0.607f, 5.7f, 0.0f}, {0.714f, 7.2f, 0.0f}, {1.14f, 7.8f, 0.0f}, {1.44f, 5.5f, 0.0f}},
+    // FP8
+    {{0.149f, 0.0f, 3.4f}, {0.209f, 0.9f, 2.7f}, {0.176f, 0.8f, 2.6f}, {0.291f, 0.9f, 2.8f}, {0.405f, 5.0f, 0.0f},
+     {0.566f, 5.5f, 0.0f}, {0.675f, 6.5f, 0.0f}, {1.09f, 7.0f, 0.0f}, {1.33f, 4.7f, 0.0f}},
+    // FP8 exact
+    {{0.238f, 0.0f, 4.6f}, {0.323f, 0.0f, 4.2f}, {0.312f, 0.0f, 4.1f}, {0.442f, 0.7f, 4.1f}, {0.745f, 5.5f, 0.0f},
+     {1.06f, 5.4f, 0.0f}, {1.32f, 7.4f, 0.0f}, {1.91f, 7.8f, 0.0f}, {2.46f, 6.9f, 0.0f}},
+};
+// The 256 x 256 kernel keeps a call unless a smaller tile is put 10% below it (where the
+// sums lie closer it was up to 10% the faster one).  Its gated form, whose epilogue runs
+// out of registers, keeps a call unless a smaller tile is put 3% below: over 80 gated
+// calls (N x K 3,072 x 3,072 to 5,376 x 14,336) the line gives up 0.02% to the best choice
+// and no call is slower than before; at 1.05 calls of several rounds lose up to 20%.
+constexpr float kKeepLarge = 0.9f, kKeepLargeGated = 0.97f;
+
+float tile_cost(int kind, int tile, int64_t M, int64_t N, int64_t K) {
+  const TileSize t = kTileSizes[tile];
+  const int64_t tiles = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
+  const int64_t cus = device_cu_count();
+  const float rounds = (float)((tiles + cus - 1) / cus);
+  // (the 256 x 256 kernel takes pairs two at a time)
+  const float pairs = (float)(tile == kTiles ? (K + 255) / 256 * 2 : (K + 127) / 128);
+  const TileCost c = kTileCosts[kind][tile];
+  return c.start + rounds * (pairs * c.per_pair + c.per_tile);
+}
+
+template <int KIND, int WM, int WN, int FM, int FN, int SLOTS>
+void launch(GemmArgs g, hipStream_t stream) {
+  typedef TileCfg<WM, WN, FM, FN, SLOTS> C;
+  g.tiles_m = (g.M + C::kM - 1) / C::kM;
+  g.tiles_n = (g.N + C::kN - 1) / C::kN;
+  g.per_xcd = (g.tiles_m * g.tiles_n + 7) / 8;
+  // the same rows per group of the tile order as the 256 x 256 kernel's
+  g.group_m = g.group_m * kTileM / C::kM;
+  gemm_tile_kernel<KIND, WM, WN, FM, FN, SLOTS><<<dim3((unsigned)g.per_xcd * 8), dim3(C::kThreads), 0, stream>>>(g);
+}
+
+template <int KIND>
+void launch_kind(int tile, const GemmArgs &g, hipStream_t stream) {
+  typedef void (*Fn)(GemmArgs, hipStream_t);
+#define XGEN_TILE_LAUNCH(WM, WN, FM, FN, S) launch<KIND, WM, WN, FM, FN, S>,
+  static constexpr Fn fns[kTiles] = {XGEN_GEMM_TILES(XGEN_TILE_LAUNCH)};
+  fns[tile](g, stream);
+}
+
+}  // namespace
+
+int choose_gemm_tile(int kind, bool gated, int64_t M, int64_t N, int64_t K) {
+  int best = kTiles;
+  float cost = (gated ? kKeepLargeGated : kKeepLarge) * tile_cost(kind, kTiles, M, N, K);
+  for (int t = 0; t < kTiles; ++t) {
+    const float c = tile_cost(kind, t, M, N, K);
+    if (c < cost) best = t, cost = c;
+  }
+  return best == kTiles ? -1 : best;
+}
+
+void launch_gemm_tile(int kind, int tile, const GemmArgs &g, hipStream_t stream) {
+  if (kind == kInt8) launch_kind<kInt8>(tile, g, stream);
+  else if (kind == kFp8) launch_kind<kFp8>(tile, g, stream);
+  else launch_kind<kFp8Exact>(tile, g, stream);
+}
+
+}  // namespace xgen
