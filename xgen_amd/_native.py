@@ -105,6 +105,11 @@ def library_path() -> Path:
     return Path(os.environ.get("XGEN_AMD_LIBRARY", default)).resolve()
 
 
+def operators_path() -> Path:
+    """The torch operators' native implementations (csrc/torch_ops.cpp), which open library_path() themselves."""
+    return Path(__file__).resolve().parent / "_lib" / "libxgen_amd_ops.so"
+
+
 def lib() -> ctypes.CDLL:
     """The loaded library (loaded on first use, once per process, under a lock)."""
     global _lib

@@ -149,7 +149,7 @@ class H3FP8Linear(nn.Module):
         x_diffusers/x_diffusers/framework/transformer/h3_npu_fusion.py:103-119).  input_activation
         does not apply here: it acts where this module quantizes its own input (quantize_input)."""
         act = _ACTIVATIONS[activation if activation is not None else self.activation]
-        out, _ = xops.scaled_mm(packed, self.weight, scale, self.weight_scale.reshape(-1), self.bias,
+        out, _ = xops.scaled_mm(packed, self.weight, scale, self.weight_scale, self.bias,
                                 out_dtype, act, False, self.accumulation == "exact")
         self.calls += 1
         return out
@@ -167,11 +167,11 @@ class H3FP8Linear(nn.Module):
             raise ValueError("forward_gate_residual: x [B,S,K] and residual [B,S,N] required")
         packed, scale = self.quantize_input(x.reshape(-1, x.shape[-1]))
         if self.accumulation == "exact":
-            branch, _ = xops.scaled_mm(packed, self.weight, scale, self.weight_scale.reshape(-1), self.bias,
+            branch, _ = xops.scaled_mm(packed, self.weight, scale, self.weight_scale, self.bias,
                                        torch.bfloat16, N.ACT_NONE, False, True)
             out = xops.gate_residual(residual, branch.reshape(residual.shape), gate_table, indices)
         else:
-            out = xops.scaled_mm_gate_residual(packed, self.weight, scale, self.weight_scale.reshape(-1), self.bias,
+            out = xops.scaled_mm_gate_residual(packed, self.weight, scale, self.weight_scale, self.bias,
                                                residual.reshape(-1, self.out_features), gate_table, indices)
         self.calls += 1
         return out.reshape(residual.shape)
@@ -185,7 +185,7 @@ class H3FP8Linear(nn.Module):
         if not matrix.shape[0]:
             return x.new_empty((*x.shape[:-1], self.out_features))
         packed, scale = self.quantize_input(matrix)
-        output, _ = xops.scaled_mm(packed, self.weight, scale, self.weight_scale.reshape(-1), bias, x.dtype,
+        output, _ = xops.scaled_mm(packed, self.weight, scale, self.weight_scale, bias, x.dtype,
                                    _ACTIVATIONS[self.activation], False, self.accumulation == "exact")
         self.calls += 1
         return output.reshape(*x.shape[:-1], self.out_features)

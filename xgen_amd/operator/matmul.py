@@ -108,7 +108,7 @@ class WeightQuantLinearModule(nn.Module):
 def quant_matmul_raw(q, scale, linear, out_dtype=torch.bfloat16, activation=N.ACT_NONE):
     """int8 GEMM of a pre-quantized activation against a WeightQuantLinearModule."""
     out, _ = xops.scaled_mm(q.reshape(-1, q.shape[-1]), linear.weight, scale.reshape(-1),
-                            linear.antiquant_scale.reshape(-1), linear.bias, out_dtype, activation, False)
+                            linear.antiquant_scale, linear.bias, out_dtype, activation, False)
     return out
 
 

@@ -61,7 +61,7 @@ def unregister_one_plus(scale: torch.Tensor) -> None:
 
 def _registered_one_plus(scale: torch.Tensor):
     """The prepared table registered for `scale` (re-prepared if `scale` was written since), or None."""
-    entry = _ONE_PLUS.get(_table_key(scale)) if _ONE_PLUS else None
+    entry = _ONE_PLUS.get(_table_key(scale))
     if entry is None or entry[0].untyped_storage().data_ptr() != scale.untyped_storage().data_ptr():
         return None
     if scale._version != entry[2]:
@@ -81,7 +81,7 @@ def norm_affine_quant(x, weight, scale, shift, indices, *, eps=1e-5, blocks=40, 
         raise RuntimeError("invalid epsilon/blocks")
     # (not under graph capture: a captured call keeps reading the table it was given, as replays
     # of the raw form would see later writes to it)
-    if not scale_is_one_plus and scale.is_cuda and not torch.cuda.is_current_stream_capturing():
+    if _ONE_PLUS and not scale_is_one_plus and scale.is_cuda and not torch.cuda.is_current_stream_capturing():
         prepared = _registered_one_plus(scale)
         if prepared is not None:
             scale, scale_is_one_plus = prepared, True

@@ -3,7 +3,9 @@
 Each operator has a CUDA-key implementation (PyTorch-ROCm exposes HIP devices
 under the CUDA key) that allocates its outputs with the caching allocator and
 launches on the current stream, and a Meta implementation with the same shape
-and dtype contract, so shapes are checkable without a GPU.  This mirrors the
+and dtype contract, so shapes are checkable without a GPU.  The CUDA-key
+implementations are native (csrc/torch_ops.cpp, _lib/libxgen_amd_ops.so), the
+SwiGLU's excepted: its silu table lives here.  This mirrors the
 reference's TORCH_LIBRARY + device + Meta registrations
 (x_base/x_base/operator/npu_fusion/f2_nq2/op_extension/nq2_queued.asc:53-61).
 Contract violations raise RuntimeError before any launch.
@@ -55,20 +57,6 @@ def _kernel_rows(t: torch.Tensor, row_align: int) -> torch.Tensor:
             and t.data_ptr() % 16 == 0):
         return t
     return t.clone(memory_format=torch.contiguous_format)
-
-
-def _aligned_flat(t: torch.Tensor) -> torch.Tensor:
-    """t contiguous with a 16-byte aligned base (copied if not)."""
-    t = t.contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone()
-
-
-def _rows_view(x: torch.Tensor) -> torch.Tensor:
-    """[..., K] -> [M, K] with unit last stride (copies only if needed)."""
-    m = x.reshape(-1, x.shape[-1])
-    if m.stride(-1) != 1 or (m.shape[0] > 1 and m.stride(0) < m.shape[1]):
-        m = m.contiguous()
-    return m
 
 
 # --------------------------------------------------------------------------- meta
@@ -233,142 +221,6 @@ def _on_gpu(*ts):
             _require(t.device == dev, "xgen_amd operators require all tensors on the same device")
 
 
-def _quantize_rows_gpu(x, out_dtype, activation=0):
-    """Per-row quantization of x, or (activation = ACT_GELU_TANH) of dtype(gelu_tanh(x)) in the same pass."""
-    _on_gpu(x)
-    q, scale = _quantize_rows_meta(x, out_dtype, activation)
-    if x.numel() == 0:
-        return q, scale
-    m = _rows_view(x)
-    fn = "xgen_quantize_rows_gelu" if activation == N.ACT_GELU_TANH else "xgen_quantize_rows"
-    st = getattr(N.lib(), fn)(N.dtype_code(x.dtype), m.data_ptr(), m.shape[0], m.shape[1], m.stride(0),
-                              N.dtype_code(out_dtype), q.data_ptr(), m.shape[1], scale.data_ptr(), N.stream_of(x))
-    N.check(st, fn)
-    return q, scale
-
-
-def _peak_common(x, fn):
-    _on_gpu(x)
-    out = _peak_meta(x)
-    _require(x.numel() > 0, f"{fn}: empty input")
-    xc = _aligned_flat(x)
-    L = N.lib()
-    ws_bytes = L.xgen_abs_peak_workspace_bytes(xc.numel())
-    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=x.device)
-    st = getattr(L, fn)(N.dtype_code(x.dtype), xc.data_ptr(), xc.numel(), out.data_ptr(), ws.data_ptr(),
-                        ws_bytes, N.stream_of(x))
-    N.check(st, fn)
-    return out
-
-
-def _peak_gpu(x):
-    return _peak_common(x, "xgen_abs_peak")
-
-
-def _tensor_scale_gpu(x):
-    return _peak_common(x, "xgen_fp8_tensor_scale")
-
-
-def _pack_gpu(x, scale):
-    _on_gpu(x, scale)
-    q = _pack_meta(x, scale)
-    if x.numel() == 0:
-        return q
-    xc = _aligned_flat(x)
-    st = N.lib().xgen_fp8_pack(N.dtype_code(x.dtype), xc.data_ptr(), xc.numel(), scale.data_ptr(), q.data_ptr(),
-                               N.stream_of(x))
-    N.check(st, "xgen_fp8_pack")
-    return q
-
-
-def _norm_gpu(x, weight, scale, shift, indices, eps, norm_kind, out_dtype, return_normed):
-    _on_gpu(x, weight, scale, shift, indices)
-    q, s, normed = _norm_meta(x, weight, scale, shift, indices, eps, norm_kind, out_dtype, return_normed)
-    if q.numel() == 0:
-        return q, s, normed
-    x, scale, shift = _kernel_rows(x, 8), _kernel_rows(scale, 8), _kernel_rows(shift, 8)
-    weight = None if weight is None else _aligned_flat(weight)
-    wcode = N.DTYPE_NONE if weight is None else N.dtype_code(weight.dtype)
-    st = N.lib().xgen_norm_affine_quant(
-        x.data_ptr(), x.shape[0], x.shape[1], x.shape[2], x.stride(0), x.stride(1), norm_kind,
-        N.ptr(weight), wcode, float(eps), scale.data_ptr(), scale.stride(0), shift.data_ptr(), shift.stride(0),
-        scale.shape[0], indices.data_ptr(), N.dtype_code(out_dtype), q.data_ptr(), s.data_ptr(),
-        normed.data_ptr() if return_normed else None, N.stream_of(x))
-    N.check(st, "xgen_norm_affine_quant")
-    return q, s, normed
-
-
-def _mm_gpu(a, w, a_scale, w_scale, bias, out_dtype, activation, return_acc, exact=False):
-    _on_gpu(a, w, a_scale, w_scale, bias)
-    out, acc = _mm_meta(a, w, a_scale, w_scale, bias, out_dtype, activation, return_acc, exact)
-    M, K = a.shape
-    Nf = w.shape[0]
-    if M == 0:
-        return out, acc
-    a, w = _kernel_rows(a, 16), _kernel_rows(w, 16)
-    a_scale = a_scale.contiguous()
-    w_scale = w_scale.contiguous()
-    bias = None if bias is None else bias.contiguous()
-    sa_stride = 1 if a_scale.numel() == M and M > 1 else 0
-    sw_stride = 1 if w_scale.numel() == Nf and Nf > 1 else 0
-    if a.dtype == torch.float8_e4m3fn:
-        fn = "xgen_scaled_mm_fp8_exact" if exact else "xgen_scaled_mm_fp8"
-    else:
-        fn = "xgen_quant_matmul_int8"
-    st = getattr(N.lib(), fn)(
-        a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), M, Nf, K, a_scale.data_ptr(), sa_stride,
-        w_scale.data_ptr(), sw_stride, N.ptr(bias), N.DTYPE_NONE if bias is None else N.dtype_code(bias.dtype),
-        activation, out.data_ptr(), N.dtype_code(out_dtype), out.stride(0),
-        acc.data_ptr() if return_acc else None, N.stream_of(a))
-    N.check(st, fn)
-    return out, acc
-
-
-def _gate_gpu(residual, branch, gate_table, indices):
-    _on_gpu(residual, branch, gate_table, indices)
-    out = _gate_meta(residual, branch, gate_table, indices)
-    if out.numel() == 0:
-        return out
-    residual, branch, gate_table = _kernel_rows(residual, 8), _kernel_rows(branch, 8), _kernel_rows(gate_table, 8)
-    indices = indices.contiguous()
-    B, S, H = residual.shape
-    st = N.lib().xgen_gate_residual(
-        residual.data_ptr(), residual.stride(0), residual.stride(1), branch.data_ptr(), branch.stride(0),
-        branch.stride(1), gate_table.data_ptr(), gate_table.stride(0), gate_table.shape[0], indices.data_ptr(),
-        B, S, H, out.data_ptr(), N.stream_of(residual))
-    N.check(st, "xgen_gate_residual")
-    return out
-
-
-def _modulate_gpu(x, scale_table, shift_table, indices, scale_is_one_plus=False):
-    _on_gpu(x, scale_table, shift_table, indices)
-    out = _modulate_meta(x, scale_table, shift_table, indices, scale_is_one_plus)
-    if out.numel() == 0:
-        return out
-    x, scale_table, shift_table = _kernel_rows(x, 8), _kernel_rows(scale_table, 8), _kernel_rows(shift_table, 8)
-    indices = indices.contiguous()
-    B, S, H = x.shape
-    st = N.lib().xgen_indexed_modulate(
-        x.data_ptr(), x.stride(0), x.stride(1), scale_table.data_ptr(), scale_table.stride(0),
-        shift_table.data_ptr(), shift_table.stride(0), scale_table.shape[0], indices.data_ptr(), B, S, H,
-        int(bool(scale_is_one_plus)), out.data_ptr(), N.stream_of(x))
-    N.check(st, "xgen_indexed_modulate")
-    return out
-
-
-def _merge_gpu(back_recv, out_dtype):
-    _on_gpu(back_recv)
-    q, scale = _merge_meta(back_recv, out_dtype)
-    if q.numel() == 0:
-        return q, scale
-    back_recv = _aligned_flat(back_recv)
-    splits, owners, seq, batch, chunk = back_recv.shape
-    st = N.lib().xgen_merge_quant(N.dtype_code(out_dtype), back_recv.data_ptr(), splits, owners, seq, batch, chunk,
-                                  q.data_ptr(), scale.data_ptr(), N.stream_of(back_recv))
-    N.check(st, "xgen_merge_quant")
-    return q, scale
-
-
 _SILU_TABLES: dict[int, torch.Tensor] = {}
 
 
@@ -402,41 +254,26 @@ def _swiglu_gpu(u, gate_first, out_dtype, scale_mode, return_act):
     return q, s, act
 
 
-def _mm_gate_gpu(a, w, a_scale, w_scale, bias, residual, gate_table, indices):
-    _on_gpu(a, w, a_scale, w_scale, bias, residual, gate_table, indices)
-    out = _mm_gate_meta(a, w, a_scale, w_scale, bias, residual, gate_table, indices)
-    M, K = a.shape
-    Nf = w.shape[0]
-    if M == 0:
-        return out
-    a, w = _kernel_rows(a, 16), _kernel_rows(w, 16)
-    a_scale, w_scale = a_scale.contiguous(), w_scale.contiguous()
-    bias = None if bias is None else bias.contiguous()
-    residual, gate_table = _kernel_rows(residual, 8), _kernel_rows(gate_table, 8)
-    indices = indices.contiguous()
-    st = N.lib().xgen_w8a8_gate_residual(
-        N.dtype_code(a.dtype), a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), M, Nf, K, a_scale.data_ptr(),
-        1 if a_scale.numel() == M and M > 1 else 0, w_scale.data_ptr(), 1 if w_scale.numel() == Nf and Nf > 1 else 0,
-        N.ptr(bias), N.DTYPE_NONE if bias is None else N.dtype_code(bias.dtype), residual.data_ptr(),
-        residual.stride(0), gate_table.data_ptr(), gate_table.stride(0), gate_table.shape[0], indices.data_ptr(),
-        indices.shape[0], out.data_ptr(), out.stride(0), N.stream_of(a))
-    N.check(st, "xgen_w8a8_gate_residual")
-    return out
-
-
-_IMPLS = {
-    "quantize_rows": (_quantize_rows_gpu, _quantize_rows_meta),
-    "abs_peak": (_peak_gpu, _peak_meta),
-    "fp8_tensor_scale": (_tensor_scale_gpu, _peak_meta),
-    "fp8_pack": (_pack_gpu, _pack_meta),
-    "norm_affine_quant": (_norm_gpu, _norm_meta),
-    "scaled_mm": (_mm_gpu, _mm_meta),
-    "gate_residual": (_gate_gpu, _gate_meta),
-    "indexed_modulate": (_modulate_gpu, _modulate_meta),
-    "merge_quant": (_merge_gpu, _merge_meta),
-    "swiglu_quant": (_swiglu_gpu, _swiglu_meta),
-    "scaled_mm_gate_residual": (_mm_gate_gpu, _mm_gate_meta),
+_META = {
+    "quantize_rows": _quantize_rows_meta,
+    "abs_peak": _peak_meta,
+    "fp8_tensor_scale": _peak_meta,
+    "fp8_pack": _pack_meta,
+    "norm_affine_quant": _norm_meta,
+    "scaled_mm": _mm_meta,
+    "gate_residual": _gate_meta,
+    "indexed_modulate": _modulate_meta,
+    "merge_quant": _merge_meta,
+    "swiglu_quant": _swiglu_meta,
+    "scaled_mm_gate_residual": _mm_gate_meta,
 }
+
+
+def _not_built(name: str, path):
+    def impl(*args, **kwargs):
+        raise RuntimeError(f"xgen_amd.{name}: native operators not found at {path}; build them with "
+                           "`python -c 'import __graft_entry__ as g; g.build()'`")
+    return impl
 
 
 def register() -> None:
@@ -447,9 +284,15 @@ def register() -> None:
     lib = torch.library.Library(NAMESPACE, "DEF")
     for name, schema in SCHEMAS.items():
         lib.define(schema)
-        gpu, meta = _IMPLS[name]
-        lib.impl(name, gpu, "CUDA")
-        lib.impl(name, meta, "Meta")
+        lib.impl(name, _META[name], "Meta")
+    lib.impl("swiglu_quant", _swiglu_gpu, "CUDA")
+    path = N.operators_path()
+    if path.is_file():
+        torch.ops.load_library(str(path))
+    else:  # no other implementation of these operators exists: calls say so
+        for name in _META:
+            if name != "swiglu_quant":
+                lib.impl(name, _not_built(name, path), "CUDA")
     _LIB = lib
 
 
