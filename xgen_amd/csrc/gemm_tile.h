@@ -14,13 +14,11 @@
 //   sub-stage 1 of pair p: MFMAs on buffer 1; the fragments of pair p + 1's
 //     sub-stage 0 are read; the DMA of pair p + SLOTS goes into pair p's slot
 //
-// so a pair's DMA has SLOTS - 1 pairs of work in front of it.  Loads past the
-// last pair are issued out of range (they write zeros to LDS), which keeps the
-// wait counts constant.
+// so a pair's DMA has SLOTS - 1 pairs of work in front of it.
 //
 // What bounds it: a tile's K steps are a serial chain, so a few hundred tokens
 // cost K / 128 steps of ~0.15 us whatever the number of workgroups below the
-// CUs' (256 x 1,024 x 1,024: 14.1 us on 256 x 256 tiles, 4 of them; 4.4 us on 128
+// CUs' (256 x 1,024 x 1,024: 14.1 us on 256 x 256 tiles, 4 of them; 4.0 us on 128
 // tiles of 32 x 64).  From about one 128 x 192 tile per CU on it is the board's
 // power: M = 1,955, N = 3,072, K = 12,288 on 256 tiles takes 62 us (2.37 PFLOP/s;
 // 104 us on 96 tiles of 256 x 256), 49 us with all operands zero, and 59 us with
@@ -29,8 +27,10 @@
 // most), which is why the 256 x 256 kernel keeps the calls that fill it.
 //
 // Epilogue: the ring is free by then; the tile's outputs are rounded into it as
-// rows, and stored from there as whole 16-byte pieces of rows (with the gated
-// residual applied at the store).
+// rows, and stored from there as whole 16-byte pieces of rows.  GATED: the gated
+// residual is applied at the store; its residual rows and table indices are read
+// in front of the last sub-stage, its gate rows one group of pieces ahead (all of
+// them read at the store: 3,906 x 3,072 x 3,072 FP8 43.2 us, 40.6 so).
 #pragma once
 
 #include "gemm_w8a8.h"
@@ -57,7 +57,7 @@ struct TileCfg {
   static_assert(kLdsBytes <= 160 * 1024, "LDS");
 };
 
-template <int KIND, int WM, int WN, int FM, int FN, int SLOTS>
+template <int KIND, int WM, int WN, int FM, int FN, int SLOTS, bool GATED>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * WM * WN, 64 * WM * WN), amdgpu_waves_per_eu(1)))
 void gemm_tile_kernel(GemmArgs p) {
   typedef TileCfg<WM, WN, FM, FN, SLOTS> C;
@@ -68,6 +68,9 @@ void gemm_tile_kernel(GemmArgs p) {
   // three slots or more: a pair's DMA loads are spread over two sub-stages (all in one queue
   // up in the address unit ahead of the MFMAs: 3% to 11% slower)
   constexpr bool kSpread = SLOTS > 2;
+  // exact kind: both operands' fragments widened once, where a wave's activation fragments
+  // fit the registers widened
+  constexpr bool kWeightsOuter = FM <= 2;
   constexpr int kFrags = KS * (FM + FN);   // fragment reads per sub-stage per wave
   __shared__ __attribute__((aligned(1024))) uint8_t smem[C::kLdsBytes];
 
@@ -148,39 +151,53 @@ void gemm_tile_kernel(GemmArgs p) {
       asm volatile("" : "+a"(acc[i][j]));
     }
 
-  // one sub-stage: its MFMAs, with the next sub-stage's fragment reads and (sub-stage 1)
-  // the DMA loads between them
-  auto sub_stage = [&](auto B, uint32_t next_slot) {
+  // one sub-stage: its MFMAs, with the next sub-stage's fragment reads (READ) and a share of
+  // a later pair's DMA loads (LOAD) between them
+  auto sub_stage = [&](auto B, auto LOAD, auto READ, uint32_t next_slot) {
     constexpr int b = decltype(B)::value;
-    if constexpr (b == 1) issue_begin();
+    constexpr bool load = decltype(LOAD)::value, read = decltype(READ)::value;
+    if constexpr (b == 1 && load) issue_begin();
     // the MFMAs are volatile asm statements: the loads written between them stay there
-    [[maybe_unused]] typename std::conditional<KIND == kFp8Exact, MfmaA<kFp8Exact>::xw_t, int>::type xw{};
+    // (the exact kind widens each activation fragment once per sub-stage and, weights
+    // outermost, each weight fragment once too)
+    [[maybe_unused]] typename std::conditional<KIND == kFp8Exact, MfmaA<kFp8Exact>::xw_t, int>::type xw[FM] = {}, ww{};
 #pragma unroll
     for (int s = 0; s < kMfmas; ++s) {
-      const int ks = s / (FM * FN), j = (s / FN) % FM, i = s % FN;
-      if constexpr (KIND == kFp8Exact) {
-        if (i == 0) xw = MfmaA<KIND>::widen_x(xf[b][ks][j]);
-        MfmaA<KIND>::mma(acc[i][j], wf[b][ks][i], xw);
+      const int ks = s / (FM * FN);
+      if constexpr (KIND == kFp8Exact && kWeightsOuter) {
+        const int i = s / FM, j = s % FM;
+        if (j == 0) ww = MfmaA<KIND>::widen_x(wf[b][ks][i]);
+        if (i == 0) xw[j] = MfmaA<KIND>::widen_x(xf[b][ks][j]);
+        MfmaA<KIND>::mma(acc[i][j], ww, xw[j]);
+      } else if constexpr (KIND == kFp8Exact) {
+        const int j = s / FN, i = s % FN;
+        if (i == 0) xw[0] = MfmaA<KIND>::widen_x(xf[b][ks][j]);
+        MfmaA<KIND>::mma(acc[i][j], wf[b][ks][i], xw[0]);
       } else {
+        const int j = (s / FN) % FM, i = s % FN;
         MfmaA<KIND>::mma(acc[i][j], wf[b][ks][i], xf[b][ks][j]);
       }
+      if constexpr (read) {
 #pragma unroll
-      for (int r = spread_first(s, kFrags, kMfmas); r < spread_first(s + 1, kFrags, kMfmas); ++r)
-        read_frag(b ^ 1, next_slot, r);
-      if constexpr (kSpread) {
+        for (int r = spread_first(s, kFrags, kMfmas); r < spread_first(s + 1, kFrags, kMfmas); ++r)
+          read_frag(b ^ 1, next_slot, r);
+      }
+      if constexpr (load && kSpread) {
         // sub-stage 1 takes the first half of a pair's loads, the next sub-stage 0 the rest
         constexpr int kFirst = (C::kLoads + 1) / 2, n = b == 1 ? kFirst : C::kLoads - kFirst, q0 = b == 1 ? 0 : kFirst;
 #pragma unroll
         for (int q = spread_first(s, n, kMfmas); q < spread_first(s + 1, n, kMfmas); ++q) issue_load(q0 + q);
-      } else if constexpr (b == 1) {
+      } else if constexpr (load && b == 1) {
 #pragma unroll
         for (int q = spread_first(s, C::kLoads, kMfmas); q < spread_first(s + 1, C::kLoads, kMfmas); ++q) issue_load(q);
       }
     }
-    if constexpr (b == (kSpread ? 0 : 1)) issue_end();
+    if constexpr (load && b == (kSpread ? 0 : 1)) issue_end();
   };
   typedef std::integral_constant<int, 0> B0;
   typedef std::integral_constant<int, 1> B1;
+  typedef std::integral_constant<bool, true> Yes;
+  typedef std::integral_constant<bool, false> No;
 
   // --- prologue: SLOTS pairs in flight, pair 0's first fragments in registers ---
 #pragma unroll
@@ -195,17 +212,69 @@ void gemm_tile_kernel(GemmArgs p) {
 #pragma unroll
   for (int r = 0; r < kFrags; ++r) read_frag(0, 0, r);
 
-  const int pairs = (p.K + 127) / 128;
-  for (int k = 0; k < pairs; ++k) {
-    sub_stage(B0(), rd_slot);
-    wait_vmcnt<(SLOTS - 2) * C::kLoads>();
+  // pairs past K are zeros: the ring is filled once at least
+  const int pairs = (p.K + 127) / 128 > SLOTS ? (p.K + 127) / 128 : SLOTS;
+  // waits for this thread's loads of the next pair (`newer` pairs were issued after them),
+  // then publishes every wave's and retires the reads of this one
+  auto publish = [&](auto NEWER) {
+    wait_vmcnt<decltype(NEWER)::value * C::kLoads>();
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     lds_barrier();
+  };
+  auto next_slot = [&]() { return rd_slot + C::kSlotBytes == C::kRing ? 0u : rd_slot + C::kSlotBytes; };
+  for (int k = 0; k < pairs - SLOTS; ++k) {
+    sub_stage(B0(), Yes(), Yes(), rd_slot);
+    publish(std::integral_constant<int, SLOTS - 2>());
     // (the DMA slot of sub-stage 1 is rd_slot: both advance once per pair)
-    const uint32_t next = rd_slot + C::kSlotBytes == C::kRing ? 0 : rd_slot + C::kSlotBytes;
-    sub_stage(B1(), next);
+    const uint32_t next = next_slot();
+    sub_stage(B1(), Yes(), Yes(), next);
     rd_slot = next;
   }
+  // the last SLOTS pairs: their loads are issued (but for the first one's share of a spread
+  // pair), so fewer and fewer stay in flight
+  auto tail = [&](auto LEFT) {  // LEFT pairs after this one
+    constexpr int left = decltype(LEFT)::value;
+    if constexpr (left == SLOTS - 1) sub_stage(B0(), Yes(), Yes(), rd_slot);
+    else sub_stage(B0(), No(), Yes(), rd_slot);
+    if constexpr (left > 0) {
+      publish(std::integral_constant<int, left - 1>());
+      const uint32_t next = next_slot();
+      sub_stage(B1(), No(), Yes(), next);
+      rd_slot = next;
+    }
+  };
+  if constexpr (SLOTS > 3) tail(std::integral_constant<int, 3>());
+  if constexpr (SLOTS > 2) tail(std::integral_constant<int, 2>());
+  tail(std::integral_constant<int, 1>());
+  tail(std::integral_constant<int, 0>());
+
+  // the gated residual's inputs, in front of the last MFMAs and the rounding: this thread's
+  // pieces of the residual rows, and their token's table indices
+  constexpr int kChunks = C::kN / 8, kPieces = C::kM * kChunks, kSteps = kPieces / C::kThreads;
+  static_assert(kPieces % C::kThreads == 0, "store split");
+  [[maybe_unused]] u32x4 res[GATED ? kSteps : 1];
+  [[maybe_unused]] u32x2 gidx[GATED ? kSteps : 1];
+  auto piece = [&](int q, uint32_t &row, uint32_t &col) {  // piece q of this thread: 8 columns of a row
+    const int c = q * C::kThreads + tid;
+    row = (uint32_t)(m0 + c / kChunks), col = (uint32_t)(n0 + c % kChunks * 8);
+    return row < (uint32_t)p.M && col < (uint32_t)p.N;
+  };
+  // (the rest, past what the registers hold beside the fragments, behind the rounding)
+  constexpr int kResAhead = kSteps <= 16 ? kSteps : 8;
+  [[maybe_unused]] auto load_res = [&](int q0, int q1) {
+    const __amdgpu_buffer_rsrc_t rres = rsrc(p.residual, p.residual_bytes), rind = rsrc(p.indices, p.seq * 8);
+#pragma unroll
+    for (int q = q0; q < q1; ++q) {
+      uint32_t row, col;
+      const bool in = piece(q, row, col);
+      const uint32_t mq = (__umulhi(row, p.seq_magic) + row) >> p.seq_shift;
+      gidx[q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rind, (row - mq * p.seq) * 8, 0, 0));
+      res[q] = __builtin_amdgcn_raw_buffer_load_b128(
+          rres, in ? (row * (uint32_t)p.ld_residual + col) * 2 : kOutOfRange, 0, 0);
+    }
+  };
+  if constexpr (GATED) load_res(0, kResAhead);
+  sub_stage(B1(), No(), No(), rd_slot);
 
   // --- epilogue --------------------------------------------------------------------
   // 24 wait states behind the last MFMAs before any accumulator is read
@@ -214,10 +283,8 @@ void gemm_tile_kernel(GemmArgs p) {
   for (int i = 0; i < FN; ++i)
 #pragma unroll
     for (int j = 0; j < FM; ++j) asm volatile("" : "+a"(acc[i][j]));
-  // the loads past the last pair may still be writing LDS, and the last fragment reads be
-  // outstanding: every wave's are done before the ring is written
-  wait_vmcnt<0>();
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  // (every DMA load has landed: the last publish waited for all; the barrier retires the
+  // other waves' fragment reads before the ring is written)
   lds_barrier();
   float *prm = reinterpret_cast<float *>(smem + C::kParamBase);  // [sa of kM][sw of kN][bias of kN]
   if (tid < C::kM) prm[tid] = sa_t;
@@ -271,52 +338,46 @@ void gemm_tile_kernel(GemmArgs p) {
     if (p.act == XGEN_ACT_NONE) round_tile(F16(), NoAct());
     else round_tile(F16(), Gelu());
   }
+  if constexpr (GATED) load_res(kResAhead, kSteps);
   __syncthreads();
 
   // rows of 16-byte pieces, consecutive lanes on consecutive pieces of a row; rows past M
   // and columns past N are dropped (N is a multiple of 16)
-  constexpr int kChunks = C::kN / 8, kPieces = C::kM * kChunks, kSteps = kPieces / C::kThreads;
-  static_assert(kPieces % C::kThreads == 0, "store split");
   const __amdgpu_buffer_rsrc_t ro = rsrc(p.out, p.out_bytes);
-  const bool gated = p.residual != nullptr;
-  const __amdgpu_buffer_rsrc_t rres = rsrc(p.residual, gated ? p.residual_bytes : 0u);
-  const __amdgpu_buffer_rsrc_t rgate = rsrc(p.gate, gated ? p.gate_bytes : 0u);
-  const __amdgpu_buffer_rsrc_t rind = rsrc(p.indices, gated ? p.seq * 8 : 0u);
   constexpr int kUnroll = kSteps % 4 == 0 ? 4 : kSteps % 3 == 0 ? 3 : kSteps % 2 == 0 ? 2 : 1;
+  [[maybe_unused]] u32x4 gt[GATED ? 2 : 1][kUnroll];  // the gate rows' pieces, one group ahead
+  [[maybe_unused]] auto load_gate = [&](int q0) {
+    const __amdgpu_buffer_rsrc_t rgate = rsrc(p.gate, p.gate_bytes);
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      uint32_t row, col;
+      const bool in = piece(q0 + u, row, col);
+      const u32x2 g = gidx[q0 + u];
+      const bool ok = g.y == 0 && g.x < (uint32_t)p.gate_rows;  // an int64 index in [0, gate_rows)
+      gt[(q0 / kUnroll) & 1][u] = __builtin_amdgcn_raw_buffer_load_b128(
+          rgate, in && ok ? (g.x * (uint32_t)p.gate_stride + col) * 2 : kOutOfRange, 0, 0);
+    }
+  };
+  if constexpr (GATED) load_gate(0);
+#pragma unroll
   for (int q0 = 0; q0 < kSteps; q0 += kUnroll) {
-    u32x4 v[kUnroll];
-    uint32_t row[kUnroll], col[kUnroll];
-    bool in[kUnroll];
+    if constexpr (GATED) {
+      __builtin_amdgcn_sched_barrier(0);  // (a later group's reads stay behind this one's: registers)
+      if (q0 + kUnroll < kSteps) load_gate(q0 + kUnroll);
+    }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       const int c = (q0 + u) * C::kThreads + tid;
-      const int r = c / kChunks, x = c % kChunks;
-      v[u] = *reinterpret_cast<const u32x4 *>(smem + r * C::kRowPitch + x * 16);
-      row[u] = (uint32_t)(m0 + r), col[u] = (uint32_t)(n0 + x * 8);
-      in[u] = row[u] < (uint32_t)p.M && col[u] < (uint32_t)p.N;
-    }
-    if (gated) {
-      u32x2 g[kUnroll];
-      u32x4 res[kUnroll], gt[kUnroll];
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-          const uint32_t mq = (__umulhi(row[u], p.seq_magic) + row[u]) >> p.seq_shift;
-        g[u] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rind, (row[u] - mq * p.seq) * 8, 0, 0));
-        res[u] = __builtin_amdgcn_raw_buffer_load_b128(
-            rres, in[u] ? (row[u] * (uint32_t)p.ld_residual + col[u]) * 2 : kOutOfRange, 0, 0);
+      uint32_t row, col;
+      const bool in = piece(q0 + u, row, col);
+      u32x4 v = *reinterpret_cast<const u32x4 *>(smem + c / kChunks * C::kRowPitch + c % kChunks * 16);
+      if constexpr (GATED) {
+        const u32x2 g = gidx[q0 + u];
+        v = g.y == 0 && g.x < (uint32_t)p.gate_rows
+                ? gate_residual8(res[q0 + u], v, gt[(q0 / kUnroll) & 1][u])
+                : u32x4{0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};  // outside the table: NaN
       }
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-          const bool ok = g[u].y == 0 && g[u].x < (uint32_t)p.gate_rows;  // an int64 index in [0, gate_rows)
-        gt[u] = __builtin_amdgcn_raw_buffer_load_b128(
-            rgate, in[u] && ok ? (g[u].x * (uint32_t)p.gate_stride + col[u]) * 2 : kOutOfRange, 0, 0);
-        v[u] = ok ? gate_residual8(res[u], v[u], gt[u])
-                  : u32x4{0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};  // outside the table: NaN
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      __builtin_amdgcn_raw_buffer_store_b128(v[u], ro, in[u] ? (row[u] * (uint32_t)p.ldo + col[u]) * 2 : kOutOfRange, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(v, ro, in ? (row * (uint32_t)p.ldo + col) * 2 : kOutOfRange, 0, 0);
     }
   }
 }

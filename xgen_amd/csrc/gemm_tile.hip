@@ -48,9 +48,10 @@ constexpr TileCost kTileCosts[3][kTiles + 1] = {
 };
 // The 256 x 256 kernel keeps a call unless a smaller tile is put 10% below it (where the
 // sums lie closer it was up to 10% the faster one).  Its gated form, whose epilogue runs
-// out of registers, keeps a call unless a smaller tile is put 3% below: over 80 gated
-// calls (N x K 3,072 x 3,072 to 5,376 x 14,336) the line gives up 0.02% to the best choice
-// and no call is slower than before; at 1.05 calls of several rounds lose up to 20%.
+// out of registers, keeps a call unless a smaller tile is put 3% below: of 80 gated
+// calls (N x K 3,072 x 3,072 to 5,376 x 14,336) none is slower there than on 256 x 256
+// (3,906 x 3,072 x 3,072 FP8: 40.6 against 45.8 us); at 1.05 calls of several rounds
+// lose up to 20%.
 constexpr float kKeepLarge = 0.9f, kKeepLargeGated = 0.97f;
 
 float tile_cost(int kind, int tile, int64_t M, int64_t N, int64_t K) {
@@ -72,7 +73,14 @@ void launch(GemmArgs g, hipStream_t stream) {
   g.per_xcd = (g.tiles_m * g.tiles_n + 7) / 8;
   // the same rows per group of the tile order as the 256 x 256 kernel's
   g.group_m = g.group_m * kTileM / C::kM;
-  gemm_tile_kernel<KIND, WM, WN, FM, FN, SLOTS><<<dim3((unsigned)g.per_xcd * 8), dim3(C::kThreads), 0, stream>>>(g);
+  const dim3 grid((unsigned)g.per_xcd * 8), block(C::kThreads);
+  if constexpr (KIND != kFp8Exact) {  // (no gated call takes the exact kind)
+    if (g.residual) {
+      gemm_tile_kernel<KIND, WM, WN, FM, FN, SLOTS, true><<<grid, block, 0, stream>>>(g);
+      return;
+    }
+  }
+  gemm_tile_kernel<KIND, WM, WN, FM, FN, SLOTS, false><<<grid, block, 0, stream>>>(g);
 }
 
 template <int KIND>

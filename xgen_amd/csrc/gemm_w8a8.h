@@ -216,6 +216,12 @@ struct MfmaA<kFp8Exact> {
     }
   }
   static __device__ __forceinline__ void mma(f32x16 &c, const i32x8 &w, const xw_t &xb) { run<false>(c, w, xb); }
+  // both operands already widened
+  static __device__ __forceinline__ void mma(f32x16 &c, const xw_t &wb, const xw_t &xb) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(wb.s[k]), "v"(xb.s[k]));
+  }
   static __device__ __forceinline__ void mma0(f32x16 &c, const i32x8 &w, const xw_t &xb) { run<true>(c, w, xb); }
   static __device__ __forceinline__ void mma(f32x16 &c, const i32x8 &w, const i32x8 &x) { run<false>(c, w, widen_x(x)); }
   static __device__ __forceinline__ void mma0(f32x16 &c, const i32x8 &w, const i32x8 &x) { run<true>(c, w, widen_x(x)); }
