@@ -28,31 +28,31 @@ constexpr TileSize kTileSizes[kTiles + 1] = {XGEN_GEMM_TILES(XGEN_TILE_SIZE){kTi
 // What a call costs on a tile, in us: start + rounds * (pairs * per_pair + per_tile),
 // rounds = tiles per CU rounded up, pairs = 128-byte steps of K.  Fitted to the times of
 // every tile on 171 shapes per kind (M 2 to 15,624; N x K from 1,024 x 1,024 to
-// 18,432 x 3,072 and 5,376 x 14,336; real-valued operands, so at the clock that the
-// power limit leaves); the choice by these sums is within 0.6% (FP8), 0.5% (INT8) and
-// 0.3% (exact) of the best tile on the average over them, and 10% at worst.  Last row:
-// the 256 x 256 kernel, whose epilogue runs under the next tile.
+// 18,432 x 3,072 and 5,376 x 14,336) on real-valued operands - at the clock that the
+// power limit leaves - and on weights that no cache holds, as between a model's layers.
+// The choice by these sums is within 0.2% of the best tile on the average over those
+// shapes, 10% at worst.  Last row: the 256 x 256 kernel, whose epilogue runs under the
+// next tile.
 struct TileCost {
   float per_pair, per_tile, start;
 };
 constexpr TileCost kTileCosts[3][kTiles + 1] = {
     // INT8
-    {{0.152f, 0.0f, 3.7f}, {0.208f, 1.0f, 2.7f}, {0.201f, 0.4f, 3.2f}, {0.286f, 1.5f, 2.4f}, {0.414f, 5.4f, 0.0f},
-     {0.607f, 5.7f, 0.0f}, {0.714f, 7.2f, 0.0f}, {1.14f, 7.8f, 0.0f}, {1.44f, 5.5f, 0.0f}},
+    {{0.219f, 0.0f, 3.6f}, {0.313f, 0.0f, 3.8f}, {0.257f, 0.0f, 3.5f}, {0.396f, 0.0f, 4.6f}, {0.504f, 3.9f, 1.6f},
+     {0.671f, 5.1f, 1.7f}, {0.762f, 6.9f, 0.0f}, {1.18f, 8.4f, 0.0f}, {1.56f, 6.7f, 0.0f}},
     // FP8
-    {{0.149f, 0.0f, 3.4f}, {0.209f, 0.9f, 2.7f}, {0.176f, 0.8f, 2.6f}, {0.291f, 0.9f, 2.8f}, {0.405f, 5.0f, 0.0f},
-     {0.566f, 5.5f, 0.0f}, {0.675f, 6.5f, 0.0f}, {1.09f, 7.0f, 0.0f}, {1.33f, 4.7f, 0.0f}},
+    {{0.217f, 0.0f, 3.6f}, {0.309f, 0.0f, 3.8f}, {0.255f, 0.0f, 3.5f}, {0.386f, 0.0f, 4.6f}, {0.495f, 3.2f, 2.2f},
+     {0.646f, 4.8f, 2.1f}, {0.722f, 6.6f, 0.2f}, {1.14f, 7.6f, 0.4f}, {1.48f, 5.4f, 1.4f}},
     // FP8 exact
-    {{0.238f, 0.0f, 4.6f}, {0.323f, 0.0f, 4.2f}, {0.312f, 0.0f, 4.1f}, {0.442f, 0.7f, 4.1f}, {0.745f, 5.5f, 0.0f},
-     {1.06f, 5.4f, 0.0f}, {1.32f, 7.4f, 0.0f}, {1.91f, 7.8f, 0.0f}, {2.46f, 6.9f, 0.0f}},
+    {{0.27f, 0.0f, 4.0f}, {0.359f, 0.0f, 3.9f}, {0.323f, 0.0f, 3.9f}, {0.485f, 0.0f, 4.9f}, {0.769f, 4.7f, 0.0f},
+     {1.07f, 4.8f, 0.0f}, {1.35f, 6.3f, 0.0f}, {1.94f, 7.6f, 0.0f}, {2.5f, 8.1f, 0.0f}},
 };
-// The 256 x 256 kernel keeps a call unless a smaller tile is put 10% below it (where the
-// sums lie closer it was up to 10% the faster one).  Its gated form, whose epilogue runs
-// out of registers, keeps a call unless a smaller tile is put 3% below: of 80 gated
-// calls (N x K 3,072 x 3,072 to 5,376 x 14,336) none is slower there than on 256 x 256
-// (3,906 x 3,072 x 3,072 FP8: 40.6 against 45.8 us); at 1.05 calls of several rounds
-// lose up to 20%.
-constexpr float kKeepLarge = 0.9f, kKeepLargeGated = 0.97f;
+// The 256 x 256 kernel keeps a call unless a smaller tile is put 4% below it: at this line
+// no fitted shape is slower than on it (at 1.0 some are, by up to 5%).  With all weights in
+// the last-level cache it would keep a few more (1,955 x 12,288 x 3,072 FP8: 69.5 us there,
+// 72.7 on 256 x 192; from memory 83.8 and 76.0).  Of 80 gated calls (N x K 3,072 x 3,072 to
+// 5,376 x 14,336) none is slower either (3,906 x 3,072 x 3,072 FP8: 40.6 against 45.8 us).
+constexpr float kKeepLarge = 0.96f;
 
 float tile_cost(int kind, int tile, int64_t M, int64_t N, int64_t K) {
   const TileSize t = kTileSizes[tile];
@@ -93,9 +93,9 @@ void launch_kind(int tile, const GemmArgs &g, hipStream_t stream) {
 
 }  // namespace
 
-int choose_gemm_tile(int kind, bool gated, int64_t M, int64_t N, int64_t K) {
+int choose_gemm_tile(int kind, int64_t M, int64_t N, int64_t K) {
   int best = kTiles;
-  float cost = (gated ? kKeepLargeGated : kKeepLarge) * tile_cost(kind, kTiles, M, N, K);
+  float cost = kKeepLarge * tile_cost(kind, kTiles, M, N, K);
   for (int t = 0; t < kTiles; ++t) {
     const float c = tile_cost(kind, t, M, N, K);
     if (c < cost) best = t, cost = c;
