@@ -142,6 +142,16 @@ int xgen_fp8_pack(int in_dtype, const void *x, int64_t numel, const float *scale
                   hipStream_t stream);
 
 /*
+ * Per-tensor FP8 quantization with no collective between its two halves
+ * (quantize_activation with group=None, x_base/x_base/operator/h3_fp8_quant.py:18-25):
+ * the scale of xgen_fp8_tensor_scale into scale[0] and the bytes of xgen_fp8_pack into q,
+ * in two launches instead of three.  q: numel bytes, 8-byte aligned.  Workspace as
+ * xgen_abs_peak's.
+ */
+int xgen_fp8_quantize_tensor(int in_dtype, const void *x, int64_t numel, void *q, float *scale,
+                             void *workspace, size_t workspace_bytes, hipStream_t stream);
+
+/*
  * Fused normalisation + AdaLN-table modulation + per-row quantization
  * (torch.ops.h3_phaa_nq2.fused, npu_fusion/f2_nq2/op_extension/nq2_queued.asc:53-61,
  *  kernel npu_fusion/f2bc/op_kernel/f2bc_kernel.asc:57-107; LayerNorm form of

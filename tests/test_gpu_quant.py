@@ -128,6 +128,25 @@ def test_pack_with_caller_scale(cuda):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("numel", [1, 7, 8, 2049, 2048 * 1024 + 5, 20_000_003])
+def test_quantize_tensor_equals_scale_then_pack(cuda, dtype, numel):
+    """fp8_quantize_tensor's scale and bytes are fp8_tensor_scale's and fp8_pack's: one workgroup to more
+    than the partial maxima's 1,024 and the resident grid, tails past the last 8 values, the peak in
+    the tail, NaN, infinity, zeros and a peak below the scale's floor."""
+    x = torch.randn(numel, generator=torch.Generator(device=cuda).manual_seed(numel), device=cuda).to(dtype)
+    views = [x, torch.zeros_like(x), (x.float() * 2.0 ** -140).to(dtype)]
+    for special in (float("nan"), float("inf"), 30000.0):
+        v = x.clone()
+        v[numel - 1] = special
+        views.append(v)
+    for v in views:
+        q, scale = xops.fp8_quantize_tensor(v)
+        want = xops.fp8_tensor_scale(v)
+        assert torch.equal(scale.view(torch.int32), want.view(torch.int32))
+        assert torch.equal(q.view(torch.uint8), xops.fp8_pack(v, want).view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_pack_infinity_in_chunk_without_nan(cuda, dtype):
     """+-Inf in 8-value chunks that hold no NaN, at power-of-two scales of the per-tensor
     kernel's form (1.0 from a peak of 448, and the FLT_MIN floor), where the fast division's

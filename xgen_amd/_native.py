@@ -51,6 +51,7 @@ SIGNATURES = {
     "xgen_fp8_tensor_scale": (_c_int, [_c_int, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "xgen_fp8_tensor_scale_noalloc": (_c_int, [_c_int, _c_ptr, _c_i64, _c_ptr, _c_ptr]),
     "xgen_fp8_pack": (_c_int, [_c_int, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr]),
+    "xgen_fp8_quantize_tensor": (_c_int, [_c_int, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "xgen_norm_affine_quant": (_c_int, [
         _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr, _c_int, _c_float,
         _c_ptr, _c_i64, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr]),

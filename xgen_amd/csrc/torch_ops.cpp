@@ -29,6 +29,7 @@ struct Api {
 #define XGEN_API(X)                                                                                         \
   X(xgen_status_string) X(xgen_last_error) X(xgen_quantize_rows) X(xgen_quantize_rows_gelu)                 \
   X(xgen_abs_peak_workspace_bytes) X(xgen_abs_peak) X(xgen_fp8_tensor_scale) X(xgen_fp8_pack)               \
+  X(xgen_fp8_quantize_tensor)                                                                               \
   X(xgen_norm_affine_quant) X(xgen_scaled_mm_fp8) X(xgen_scaled_mm_fp8_exact) X(xgen_quant_matmul_int8)     \
   X(xgen_gate_residual) X(xgen_indexed_modulate) X(xgen_merge_quant) X(xgen_w8a8_gate_residual)
 #define XGEN_FIELD(f) decltype(&::f) f;
@@ -180,6 +181,22 @@ Tensor fp8_pack(const Tensor &x, const Tensor &scale) {
                             q.data_ptr(), stream_of(x)),
         "xgen_fp8_pack");
   return q;
+}
+
+std::tuple<Tensor, Tensor> fp8_quantize_tensor(const Tensor &x) {
+  const char *fn = "xgen_fp8_quantize_tensor";
+  on_gpu(x);
+  TORCH_CHECK(is_half(x), "abs_peak: BF16/F16 input required");
+  TORCH_CHECK(x.numel() > 0, "xgen_fp8_tensor_scale: empty input");
+  const c10::DeviceGuard guard(x.device());
+  Tensor q = empty(x.sizes(), at::kFloat8_e4m3fn, x), scale = empty({}, at::kFloat, x);
+  const Tensor xc = aligned_flat(x);
+  const size_t bytes = api().xgen_abs_peak_workspace_bytes(xc.numel());
+  Tensor ws = empty({(int64_t)bytes}, at::kByte, x);
+  check(api().xgen_fp8_quantize_tensor(dtype_code(x.scalar_type()), xc.data_ptr(), xc.numel(), q.data_ptr(),
+                                       scale.data_ptr<float>(), ws.data_ptr(), bytes, stream_of(x)),
+        fn);
+  return {q, scale};
 }
 
 std::tuple<Tensor, Tensor, Tensor> norm_affine_quant(const Tensor &x_in, const OptTensor &weight, const Tensor &scale_in,
@@ -391,6 +408,7 @@ TORCH_LIBRARY_IMPL(xgen_amd, CUDA, m) {
   m.impl("abs_peak", abs_peak);
   m.impl("fp8_tensor_scale", fp8_tensor_scale);
   m.impl("fp8_pack", fp8_pack);
+  m.impl("fp8_quantize_tensor", fp8_quantize_tensor);
   m.impl("norm_affine_quant", norm_affine_quant);
   m.impl("scaled_mm", scaled_mm);
   m.impl("scaled_mm_gate_residual", scaled_mm_gate_residual);

@@ -14,10 +14,11 @@ from ..ops import xops
 
 def quantize_activation(x: torch.Tensor, group=None):
     """Per-tensor FP8 quantization -> (e4m3fn tensor shaped like x, float32 0-dim scale)."""
+    if group is None:
+        return xops.fp8_quantize_tensor(x)
+    import torch.distributed as dist
     scale = xops.fp8_tensor_scale(x)
-    if group is not None:
-        import torch.distributed as dist
-        dist.all_reduce(scale, op=dist.ReduceOp.MAX, group=group)
+    dist.all_reduce(scale, op=dist.ReduceOp.MAX, group=group)
     return xops.fp8_pack(x, scale), scale
 
 

@@ -24,6 +24,7 @@ SCHEMAS = {
     "abs_peak": "abs_peak(Tensor x) -> Tensor",
     "fp8_tensor_scale": "fp8_tensor_scale(Tensor x) -> Tensor",
     "fp8_pack": "fp8_pack(Tensor x, Tensor scale) -> Tensor",
+    "fp8_quantize_tensor": "fp8_quantize_tensor(Tensor x) -> (Tensor, Tensor)",
     "norm_affine_quant": (
         "norm_affine_quant(Tensor x, Tensor? weight, Tensor scale, Tensor shift, Tensor indices, "
         "float eps, int norm_kind, ScalarType out_dtype, bool return_normed) -> (Tensor, Tensor, Tensor)"),
@@ -78,6 +79,12 @@ def _pack_meta(x, scale):
     _require(x.dtype in (torch.bfloat16, torch.float16), "fp8_pack: BF16/F16 input required")
     _require(scale.dtype == torch.float32 and scale.numel() == 1, "fp8_pack: one float32 scale required")
     return torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device)
+
+
+def _quantize_tensor_meta(x):
+    """(fp8_pack(x, s), s) with s = fp8_tensor_scale(x)."""
+    scale = _peak_meta(x)
+    return _pack_meta(x, scale), scale
 
 
 def _norm_check(x, weight, scale, shift, indices, eps, norm_kind, out_dtype):
@@ -259,6 +266,7 @@ _META = {
     "abs_peak": _peak_meta,
     "fp8_tensor_scale": _peak_meta,
     "fp8_pack": _pack_meta,
+    "fp8_quantize_tensor": _quantize_tensor_meta,
     "norm_affine_quant": _norm_meta,
     "scaled_mm": _mm_meta,
     "gate_residual": _gate_meta,
