@@ -243,6 +243,9 @@ void gemm_tile_kernel(GemmArgs p) {
       rd_slot = next;
     }
   };
+  static_assert(SLOTS >= 2 && SLOTS <= 6, "tail");
+  if constexpr (SLOTS > 5) tail(std::integral_constant<int, 5>());
+  if constexpr (SLOTS > 4) tail(std::integral_constant<int, 4>());
   if constexpr (SLOTS > 3) tail(std::integral_constant<int, 3>());
   if constexpr (SLOTS > 2) tail(std::integral_constant<int, 2>());
   tail(std::integral_constant<int, 1>());
