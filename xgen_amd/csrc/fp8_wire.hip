@@ -80,9 +80,11 @@ __device__ __forceinline__ T ld_global(const void *p) {
   if constexpr (NT) return __builtin_nontemporal_load((const XGEN_GLOBAL T *)p);
   else return *(const XGEN_GLOBAL T *)p;
 }
-template <typename T>
+// NT: non-temporal store, for outputs that a call's footprint pushes past that cache.
+template <bool NT = false, typename T>
 __device__ __forceinline__ void st_global(void *p, const T &v) {
-  *(XGEN_GLOBAL T *)p = v;
+  if constexpr (NT) __builtin_nontemporal_store(v, (XGEN_GLOBAL T *)p);
+  else *(XGEN_GLOBAL T *)p = v;
 }
 // Dword pairs at addresses that are only 4-byte aligned (wire rows).
 __device__ __forceinline__ u32x2 ld_global_a4x2(const void *p) { return *(const XGEN_GLOBAL u32x2_a4 *)p; }
@@ -364,7 +366,7 @@ __device__ __forceinline__ void decode4(uint32_t b, float s, float (&v)[4]) {
   v[0] = lo.x * s, v[1] = lo.y * s, v[2] = hi.x * s, v[3] = hi.y * s;
 }
 
-template <int OT, int E, bool ALIGNED, int C, bool STRIDED>
+template <int OT, int E, bool ALIGNED, int C, bool STRIDED, bool NT>
 __global__ __launch_bounds__(kThreads) void wire_decode_kernel(DecodeArgs a) {
   constexpr int kOb = Elem<OT>::kBytes;
   const int lanes = 1 << a.log2_lanes;
@@ -434,7 +436,7 @@ __global__ __launch_bounds__(kThreads) void wire_decode_kernel(DecodeArgs a) {
           else
             o = u32x4{pack_f16x2(v0[0], v0[1]), pack_f16x2(v0[2], v0[3]), pack_f16x2(v1[0], v1[1]),
                       pack_f16x2(v1[2], v1[3])};
-          st_global(out + (int64_t)e0 * kOb, o);
+          st_global<NT>(out + (int64_t)e0 * kOb, o);
         } else {
           float v[4];
           decode4(cur.b[j][0], cur.s, v);
@@ -501,18 +503,33 @@ struct EncodeK {
 };
 // Non-temporal input loads: 8% faster (H3 Q/K/V, 288 MB in + 149 MB out) once
 // a call's footprint exceeds the last-level cache; the decoder, whose input is
-// the smaller side, gains nothing from them.
+// the smaller side, gains nothing from them, but from non-temporal 16-byte output
+// stores at the same line: the outputs then leave the wire, written just before,
+// in the cache.  H3 Q/K/V, decode alone 82.4 -> 78.9 us, after its encode 83 -> 63 (the
+// pair 166 -> 145), the gather's strided stores 88.6 -> 65.4.  Below the line a decode
+// alone gains as well (3,906 tokens: 22.5 -> 17.5 us), but what reads its outputs next
+// finds them in memory instead of the cache and loses more (decode and one read of the
+// outputs 46.0 -> 49.3 us; at 15,624 tokens 169.3 -> 167.3).
 template <int DT, int E, bool ALIGNED, int C>
 struct EncodeNtK {
   static constexpr auto kernel = wire_encode_kernel<DT, E, ALIGNED, C, true>;
 };
 template <int OT, int E, bool ALIGNED, int C>
 struct DecodeK {
-  static constexpr auto kernel = wire_decode_kernel<OT, E, ALIGNED, C, false>;
+  static constexpr auto kernel = wire_decode_kernel<OT, E, ALIGNED, C, false, false>;
 };
 template <int OT, int E, bool ALIGNED, int C>
 struct DecodeStridedK {
-  static constexpr auto kernel = wire_decode_kernel<OT, E, ALIGNED, C, true>;
+  static constexpr auto kernel = wire_decode_kernel<OT, E, ALIGNED, C, true, false>;
+};
+// (only the 16-byte stores of 8 values have a non-temporal form)
+template <int OT, int E, bool ALIGNED, int C>
+struct DecodeNtK {
+  static constexpr auto kernel = wire_decode_kernel<OT, E, ALIGNED, C, false, E == 8>;
+};
+template <int OT, int E, bool ALIGNED, int C>
+struct DecodeStridedNtK {
+  static constexpr auto kernel = wire_decode_kernel<OT, E, ALIGNED, C, true, E == 8>;
 };
 
 bool is_wire_dtype(int dt) { return dt == XGEN_DTYPE_BF16 || dt == XGEN_DTYPE_F16 || dt == XGEN_DTYPE_F32; }
@@ -696,8 +713,15 @@ int wire_decode(const char *fn, int out_dtype, int streams, const void *wire, in
   // chunks of 8 values (16-byte stores of 16-bit output) or 4 (16-byte f32 / 8-byte stores)
   const Shape sh = pick_shape((int)width, vec16 ? 8 : 4, kDecodeChunks);
   a.log2_lanes = sh.log2_lanes;
-  if (dst_strides) launch_decode<DecodeStridedK>(out_dtype, vec, a, sh, stream);
-  else launch_decode<DecodeK>(out_dtype, vec, a, sh, stream);
+  // bytes read and written by the call
+  const bool nt = (int64_t)a.g.total * (width * (eb + 1) + 4) > kLastLevelCacheBytes;
+  if (dst_strides) {
+    if (nt) launch_decode<DecodeStridedNtK>(out_dtype, vec, a, sh, stream);
+    else launch_decode<DecodeStridedK>(out_dtype, vec, a, sh, stream);
+  } else {
+    if (nt) launch_decode<DecodeNtK>(out_dtype, vec, a, sh, stream);
+    else launch_decode<DecodeK>(out_dtype, vec, a, sh, stream);
+  }
   return launch_status(fn);
 }
 
