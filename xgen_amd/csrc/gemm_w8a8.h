@@ -29,7 +29,7 @@ struct GemmArgs {
   void *acc_out;
   int tiles_m, tiles_n, per_xcd;
   int group_m;  // tile-rows per group of the tile order
-  int kt4;      // stages per tile of the one-wave-per-SIMD kernel (a multiple of 4)
+  int kt4;      // stages per tile of the 256 x 256 kernel (a multiple of 4)
   uint32_t out_bytes;  // bytes of the output rows: (M - 1) * ldo * 2 + N * 2
   uint32_t a_bytes, w_bytes;
   // gated residual epilogue (GATED kernels only)
@@ -155,13 +155,14 @@ __device__ __forceinline__ void tile_origin(int pid, int tiles_m, int tiles_n, i
 // Loads [first(s), first(s + 1)) of n loads spread over `slots` MFMA slots.
 __host__ __device__ constexpr int spread_first(int s, int n, int slots) { return (s * n + slots - 1) / slots; }
 
-// The MFMAs of the one-wave-per-SIMD kernel, with their accumulators pinned
+// The kernels' MFMAs, with their accumulators pinned
 // to AGPRs ("+a"): left to the register allocator, 256 accumulators plus the
 // double-buffered fragments are shuffled between the register files and
 // spilled.  The compiler sees these as opaque, so the kernel itself keeps the
 // MFMA result hazards: a tile's first MFMA per accumulator adds an
-// inline-constant zero (no VALU writes to accumulators at all), and the
-// epilogue reads accumulators only after mfma_drain's wait states behind the
+// inline-constant zero (no VALU writes to accumulators at all; the tile kernels
+// zero them long before the first MFMA), and the
+// epilogue reads accumulators only after 24 wait states behind the
 // tile's last MFMA.  Operand registers are written only by LDS loads, which
 // the compiler's wait counts order before the MFMA that reads them; a buffer
 // is reloaded only after the barrier that follows its last MFMA.

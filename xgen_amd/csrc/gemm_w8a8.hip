@@ -31,6 +31,9 @@
 // accumulator rows are 4 consecutive output features: the epilogue writes 8
 // contiguous bytes per lane per group.
 //
+// Calls that leave compute units idle at 256x256 run on smaller tiles, with the
+// same bits (gemm_tile.hip chooses, gemm_tile.h is their kernel).
+//
 // Workgroup -> tile mapping: the dispatcher places consecutive workgroup ids
 // on the 8 XCDs round-robin; ids are remapped so each XCD owns a contiguous
 // range of tiles, walked in groups of 8 tile-rows, so concurrently running
