@@ -41,6 +41,7 @@
 // strides from a table in LDS.  The row max is a DPP / ds_swizzle butterfly
 // inside the group.
 #include "fastdiv.h"
+#include "wire_policy.h"
 #include "xgen_common.h"
 
 namespace xgen {
@@ -504,12 +505,7 @@ struct EncodeK {
 // Non-temporal input loads: 8% faster (H3 Q/K/V, 288 MB in + 149 MB out) once
 // a call's footprint exceeds the last-level cache; the decoder, whose input is
 // the smaller side, gains nothing from them, but from non-temporal 16-byte output
-// stores at the same line: the outputs then leave the wire, written just before,
-// in the cache.  H3 Q/K/V, decode alone 82.4 -> 78.9 us, after its encode 83 -> 63 (the
-// pair 166 -> 145), the gather's strided stores 88.6 -> 65.4.  Below the line a decode
-// alone gains as well (3,906 tokens: 22.5 -> 17.5 us), but what reads its outputs next
-// finds them in memory instead of the cache and loses more (decode and one read of the
-// outputs 46.0 -> 49.3 us; at 15,624 tokens 169.3 -> 167.3).
+// stores (wire_policy.h: which calls, and what they measured).
 template <int DT, int E, bool ALIGNED, int C>
 struct EncodeNtK {
   static constexpr auto kernel = wire_encode_kernel<DT, E, ALIGNED, C, true>;
@@ -713,8 +709,12 @@ int wire_decode(const char *fn, int out_dtype, int streams, const void *wire, in
   // chunks of 8 values (16-byte stores of 16-bit output) or 4 (16-byte f32 / 8-byte stores)
   const Shape sh = pick_shape((int)width, vec16 ? 8 : 4, kDecodeChunks);
   a.log2_lanes = sh.log2_lanes;
-  // bytes read and written by the call
-  const bool nt = (int64_t)a.g.total * (width * (eb + 1) + 4) > kLastLevelCacheBytes;
+  uint64_t bits = 0;
+  for (int s = 0; s < streams; ++s) bits |= reinterpret_cast<uintptr_t>(dst[s]);
+  for (int d = 0; d < 4; ++d) bits |= (uint64_t)a.dst_st[d];
+  // (bytes read and written by the call)
+  const bool nt = decode_stores_non_temporal((int64_t)a.g.total * (width * (eb + 1) + 4), kLastLevelCacheBytes,
+                                             a.dst_row_bytes, 1 << sh.log2_lanes, dst_strides != nullptr, bits);
   if (dst_strides) {
     if (nt) launch_decode<DecodeStridedNtK>(out_dtype, vec, a, sh, stream);
     else launch_decode<DecodeStridedK>(out_dtype, vec, a, sh, stream);
