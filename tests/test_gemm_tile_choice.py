@@ -1,0 +1,44 @@
+"""The output tile that a W8A8 GEMM call runs on (xgen_amd/csrc/gemm_tile.hip: choose_gemm_tile), asked of
+the built library on the host.  Without a device it counts 256 CUs, an MI355X's."""
+import ctypes
+
+import pytest
+
+KINDS = {"int8": 0, "fp8": 1, "fp8_exact": 2}
+LARGE = (256, 256)
+
+
+def tile_choice(path, kind, M, Nf, K, gated=False):
+    fn = ctypes.CDLL(str(path)).xgen_gemm_tile_choice
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_int] + [ctypes.c_int64] * 3 + [ctypes.c_int,
+                                                                                  ctypes.POINTER(ctypes.c_int)]
+    n = ctypes.c_int()
+    m = fn(KINDS[kind], M, Nf, K, int(gated), ctypes.byref(n))
+    return m, n.value
+
+
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("kind", sorted(KINDS))
+@pytest.mark.parametrize("K", [16, 64, 128, 256])
+@pytest.mark.parametrize("M,Nf", [(8192, 9216), (15624, 3072), (15624, 18432), (31248, 9216), (66048, 16384)])
+def test_many_rows_of_short_k_stay_on_the_large_kernel(built_library, M, Nf, K, kind, gated):
+    """A smaller tile takes as many K steps as it has slots, whatever K: 32 x 128 measured up to 3.8
+    times the 256 x 256 kernel's time on these."""
+    assert tile_choice(built_library, kind, M, Nf, K, gated) == LARGE
+
+
+@pytest.mark.parametrize("kind,M,Nf,K,gated,tile", [
+    ("fp8_exact", 256, 1024, 1024, False, (32, 64)),     # latency: as many workgroups as there are CUs
+    ("int8", 2, 18432, 3072, False, (32, 128)),
+    ("fp8_exact", 1003, 3072, 3072, False, (128, 128)),
+    ("fp8", 1955, 12288, 3072, False, (256, 192)),
+    ("fp8", 1955, 3072, 12288, False, (128, 192)),
+    ("fp8", 3906, 3072, 3072, True, (256, 192)),
+    ("fp8", 15624, 9216, 3072, False, LARGE),
+    ("int8", 15624, 12288, 3072, False, LARGE),
+    ("fp8", 15624, 3072, 3072, True, LARGE),
+    ("fp8_exact", 1955, 18432, 64, False, LARGE),        # short K: 10% below the large kernel or not at all
+    ("fp8_exact", 100, 1024, 64, False, (32, 128)),      # few rows of short K leave it idle
+])
+def test_choice(built_library, kind, M, Nf, K, gated, tile):
+    assert tile_choice(built_library, kind, M, Nf, K, gated) == tile

@@ -23,19 +23,20 @@ namespace {
 
 constexpr int kTiles = 8;
 struct TileSize {
-  int m, n;
+  int m, n, slots;
 };
-#define XGEN_TILE_SIZE(WM, WN, FM, FN, S) {TileCfg<WM, WN, FM, FN, S>::kM, TileCfg<WM, WN, FM, FN, S>::kN},
-constexpr TileSize kTileSizes[kTiles + 1] = {XGEN_GEMM_TILES(XGEN_TILE_SIZE){kTileM, kTileN}};
+#define XGEN_TILE_SIZE(WM, WN, FM, FN, S) {TileCfg<WM, WN, FM, FN, S>::kM, TileCfg<WM, WN, FM, FN, S>::kN, S},
+constexpr TileSize kTileSizes[kTiles + 1] = {XGEN_GEMM_TILES(XGEN_TILE_SIZE){kTileM, kTileN, 0}};
 
 // What a call costs on a tile, in us: start + rounds * (pairs * per_pair + per_tile),
-// rounds = tiles per CU rounded up, pairs = 128-byte steps of K.  Fitted to the times of
-// every tile on 171 shapes per kind (M 2 to 15,624; N x K from 1,024 x 1,024 to
-// 18,432 x 3,072 and 5,376 x 14,336) on real-valued operands - at the clock that the
-// power limit leaves - and on weights that no cache holds, as between a model's layers.
-// The choice by these sums is within 0.2% (exact kind 0.4%) of the best tile on the average
-// over those shapes, 9% at worst.  Last row: the 256 x 256 kernel, whose epilogue runs under the
-// next tile.
+// rounds = tiles per CU rounded up, pairs = the 128-byte steps of K that the kernel takes, at
+// least its SLOTS (31,248 x 18,432 x 64 FP8, one step: 823 us on 32 x 128, which takes four, 239
+// on 256 x 256).  Fitted to the times of every tile on 171 shapes per kind (M 2 to 15,624; N x K
+// from 1,024 x 1,024 to 18,432 x 3,072 and 5,376 x 14,336) on real-valued operands - at the clock
+// that the power limit leaves - and on weights that no cache holds, as between a model's layers.
+// Over 1,916 more (M 2 to 31,248, N 16 to 18,432, K 16 to 14,336) the choice by these sums and
+// the lines below is within 0.7% of the best tile on the average.  Last row: the 256 x 256
+// kernel, whose epilogue runs under the next tile.
 struct TileCost {
   float per_pair, per_tile, start;
 };
@@ -50,12 +51,15 @@ constexpr TileCost kTileCosts[3][kTiles + 1] = {
     {{0.266f, 0.0f, 4.0f}, {0.363f, 0.0f, 3.9f}, {0.367f, 2.2f, 1.5f}, {0.492f, 3.0f, 1.2f}, {0.771f, 4.7f, 0.0f},
      {1.06f, 4.8f, 0.0f}, {1.35f, 6.4f, 0.0f}, {1.92f, 7.8f, 0.0f}, {2.49f, 7.7f, 0.0f}},
 };
-// The 256 x 256 kernel keeps a call unless a smaller tile is put 4% below it: at this line
-// no fitted shape is slower than on it (at 1.0 some are, by up to 5%).  With all weights in
-// the last-level cache it would keep a few more (1,955 x 12,288 x 3,072 FP8: 69.5 us there,
-// 72.7 on 256 x 192; from memory 83.8 and 76.0).  Of 80 gated calls (N x K 3,072 x 3,072 to
-// 5,376 x 14,336) none is slower either (3,906 x 3,072 x 3,072 FP8: 40.6 against 45.8 us).
-constexpr float kKeepLarge = 0.96f;
+// The 256 x 256 kernel keeps a call unless a smaller tile is put 4% below it.  On short K, where
+// the sums put its epilogue too high, 10%: up to K = 512, and against the tiles from 128 x 192 on up
+// to 1,024 (at 4%, 1,955 x 18,432 x 64 exact: 37.6 us on 256 x 192, 31.6 there).  So 35 of 5,748
+// calls on those shapes are more than 3% slower than on it, 9% at most.  A gated call's epilogue is what a smaller tile saves most: 4% for all of them, and of 840
+// none is slower (3,906 x 3,072 x 3,072 FP8: 40.6 against 45.8 us).
+float keep_large(int tile, int64_t K, bool gated) {
+  const int64_t short_k = kTileSizes[tile].m * kTileSizes[tile].n >= 128 * 192 ? 1024 : 512;
+  return !gated && K <= short_k ? 0.90f : 0.96f;
+}
 
 float tile_cost(int kind, int tile, int64_t M, int64_t N, int64_t K) {
   const TileSize t = kTileSizes[tile];
@@ -63,7 +67,8 @@ float tile_cost(int kind, int tile, int64_t M, int64_t N, int64_t K) {
   const int64_t cus = device_cu_count();
   const float rounds = (float)((tiles + cus - 1) / cus);
   // (the 256 x 256 kernel takes pairs two at a time)
-  const float pairs = (float)(tile == kTiles ? (K + 255) / 256 * 2 : (K + 127) / 128);
+  const int64_t steps = tile == kTiles ? (K + 255) / 256 * 2 : (K + 127) / 128;
+  const float pairs = (float)(steps > t.slots ? steps : t.slots);
   const TileCost c = kTileCosts[kind][tile];
   return c.start + rounds * (pairs * c.per_pair + c.per_tile);
 }
@@ -96,14 +101,15 @@ void launch_kind(int tile, const GemmArgs &g, hipStream_t stream) {
 
 }  // namespace
 
-int choose_gemm_tile(int kind, int64_t M, int64_t N, int64_t K) {
-  int best = kTiles;
-  float cost = kKeepLarge * tile_cost(kind, kTiles, M, N, K);
+int choose_gemm_tile(int kind, int64_t M, int64_t N, int64_t K, bool gated) {
+  const float large = tile_cost(kind, kTiles, M, N, K);
+  int best = -1;
+  float cost = large;
   for (int t = 0; t < kTiles; ++t) {
     const float c = tile_cost(kind, t, M, N, K);
-    if (c < cost) best = t, cost = c;
+    if (c < cost && c < keep_large(t, K, gated) * large) best = t, cost = c;
   }
-  return best == kTiles ? -1 : best;
+  return best;
 }
 
 void launch_gemm_tile(int kind, int tile, const GemmArgs &g, hipStream_t stream) {
@@ -113,3 +119,12 @@ void launch_gemm_tile(int kind, int tile, const GemmArgs &g, hipStream_t stream)
 }
 
 }  // namespace xgen
+
+// The rows (and columns, in *n) of the output tiles that a call runs on.  Not part of the C ABI: for
+// the tests, which choose their shapes by it.
+extern "C" int xgen_gemm_tile_choice(int kind, int64_t M, int64_t N, int64_t K, int gated, int *n) {
+  const int tile = xgen::choose_gemm_tile(kind, M, N, K, gated != 0);
+  const xgen::TileSize t = xgen::kTileSizes[tile < 0 ? xgen::kTiles : tile];
+  *n = t.n;
+  return t.m;
+}
