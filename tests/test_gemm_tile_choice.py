@@ -8,12 +8,12 @@ KINDS = {"int8": 0, "fp8": 1, "fp8_exact": 2}
 LARGE = (256, 256)
 
 
-def tile_choice(path, kind, M, Nf, K, gated=False):
+def tile_choice(path, kind, M, Nf, K, gated=False, accumulators=False):
     fn = ctypes.CDLL(str(path)).xgen_gemm_tile_choice
-    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_int] + [ctypes.c_int64] * 3 + [ctypes.c_int,
-                                                                                  ctypes.POINTER(ctypes.c_int)]
+    fn.restype = ctypes.c_int
+    fn.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3 + [ctypes.c_int] * 2 + [ctypes.POINTER(ctypes.c_int)]
     n = ctypes.c_int()
-    m = fn(KINDS[kind], M, Nf, K, int(gated), ctypes.byref(n))
+    m = fn(KINDS[kind], M, Nf, K, int(gated), int(accumulators), ctypes.byref(n))
     return m, n.value
 
 
@@ -42,3 +42,14 @@ def test_many_rows_of_short_k_stay_on_the_large_kernel(built_library, M, Nf, K, 
 ])
 def test_choice(built_library, kind, M, Nf, K, gated, tile):
     assert tile_choice(built_library, kind, M, Nf, K, gated) == tile
+
+
+@pytest.mark.parametrize("kind,M,Nf,K,plain,accumulators", [
+    ("fp8_exact", 15624, 5376, 384, (256, 192), LARGE),  # the accumulators' stores: 228 us on 256 x 192, 148 there
+    ("fp8", 13032, 5376, 7168, (256, 128), LARGE),
+    ("fp8", 1955, 12288, 3072, (256, 192), (256, 192)),
+    ("fp8_exact", 1003, 3072, 3072, (128, 128), (128, 128)),
+])
+def test_choice_with_accumulators(built_library, kind, M, Nf, K, plain, accumulators):
+    assert tile_choice(built_library, kind, M, Nf, K) == plain
+    assert tile_choice(built_library, kind, M, Nf, K, accumulators=True) == accumulators

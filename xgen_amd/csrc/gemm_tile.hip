@@ -55,8 +55,12 @@ constexpr TileCost kTileCosts[3][kTiles + 1] = {
 // the sums put its epilogue too high, 10%: up to K = 512, and against the tiles from 128 x 192 on up
 // to 1,024 (at 4%, 1,955 x 18,432 x 64 exact: 37.6 us on 256 x 192, 31.6 there).  So 35 of 5,748
 // calls on those shapes are more than 3% slower than on it, 9% at most.  A gated call's epilogue is what a smaller tile saves most: 4% for all of them, and of 840
-// none is slower (3,906 x 3,072 x 3,072 FP8: 40.6 against 45.8 us).
-float keep_large(int tile, int64_t K, bool gated) {
+// none is slower (3,906 x 3,072 x 3,072 FP8: 40.6 against 45.8 us).  A call that stores its
+// accumulators stores three times the bytes, on the 256-row tiles all at the end: 15% for them (at
+// the lines above, 15,624 x 5,376 x 384 exact: 228 us on 256 x 192, 148 on the large kernel, and 44
+// of 1,776 calls more than 3% slower than on it; so 18, most of them under K = 1,024, 17% at most).
+float keep_large(int tile, int64_t K, bool gated, bool accumulators) {
+  if (accumulators && kTileSizes[tile].m == 256) return 0.85f;
   const int64_t short_k = kTileSizes[tile].m * kTileSizes[tile].n >= 128 * 192 ? 1024 : 512;
   return !gated && K <= short_k ? 0.90f : 0.96f;
 }
@@ -101,13 +105,13 @@ void launch_kind(int tile, const GemmArgs &g, hipStream_t stream) {
 
 }  // namespace
 
-int choose_gemm_tile(int kind, int64_t M, int64_t N, int64_t K, bool gated) {
+int choose_gemm_tile(int kind, int64_t M, int64_t N, int64_t K, bool gated, bool accumulators) {
   const float large = tile_cost(kind, kTiles, M, N, K);
   int best = -1;
   float cost = large;
   for (int t = 0; t < kTiles; ++t) {
     const float c = tile_cost(kind, t, M, N, K);
-    if (c < cost && c < keep_large(t, K, gated) * large) best = t, cost = c;
+    if (c < cost && c < keep_large(t, K, gated, accumulators) * large) best = t, cost = c;
   }
   return best;
 }
@@ -122,8 +126,8 @@ void launch_gemm_tile(int kind, int tile, const GemmArgs &g, hipStream_t stream)
 
 // The rows (and columns, in *n) of the output tiles that a call runs on.  Not part of the C ABI: for
 // the tests, which choose their shapes by it.
-extern "C" int xgen_gemm_tile_choice(int kind, int64_t M, int64_t N, int64_t K, int gated, int *n) {
-  const int tile = xgen::choose_gemm_tile(kind, M, N, K, gated != 0);
+extern "C" int xgen_gemm_tile_choice(int kind, int64_t M, int64_t N, int64_t K, int gated, int accumulators, int *n) {
+  const int tile = xgen::choose_gemm_tile(kind, M, N, K, gated != 0, accumulators != 0);
   const xgen::TileSize t = xgen::kTileSizes[tile < 0 ? xgen::kTiles : tile];
   *n = t.n;
   return t.m;

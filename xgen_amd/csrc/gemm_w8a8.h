@@ -47,7 +47,7 @@ struct GemmArgs {
 enum Kind { kInt8 = 0, kFp8 = 1, kFp8Exact = 2 };
 
 // The smaller tile that a call runs on, or -1: the 256 x 256 kernel (gemm_tile.hip).
-int choose_gemm_tile(int kind, int64_t M, int64_t N, int64_t K, bool gated);
+int choose_gemm_tile(int kind, int64_t M, int64_t N, int64_t K, bool gated, bool accumulators);
 // Launches the call on that tile.  g: filled as for the 256 x 256 kernel.
 void launch_gemm_tile(int kind, int tile, const GemmArgs &g, hipStream_t stream);
 

@@ -735,7 +735,7 @@ int gemm_entry(const char *fn, const void *a, int64_t lda, const void *w, int64_
   g.out_bytes = (uint32_t)out_bytes;
   g.act = activation;
   g.out_dtype = out_dtype;
-  const int tile = choose_gemm_tile(KIND, M, N, K, gated);
+  const int tile = choose_gemm_tile(KIND, M, N, K, gated, acc_out != nullptr);
   if (tile >= 0) {
     launch_gemm_tile(KIND, tile, g, stream);
     return launch_status(fn);
