@@ -14,10 +14,10 @@ def pytest_configure(config):
 
 @pytest.fixture(scope="session")
 def built_library():
-    """Path of libxgen_amd.so, building it (hipcc cross-compiles) if absent."""
+    """Path of libxgen_amd.so, building it (hipcc cross-compiles) and the native operators if either is absent."""
     from xgen_amd import _native
     path = _native.library_path()
-    if not path.is_file():
+    if not (path.is_file() and _native.operators_path().is_file()):
         from xgen_amd import _build
         _build.build()
     return path

@@ -12,6 +12,8 @@ Contract violations raise RuntimeError before any launch.
 """
 from __future__ import annotations
 
+import threading
+
 import torch
 
 from . import _native as N
@@ -277,15 +279,43 @@ _META = {
 }
 
 
-def _not_built(name: str, path):
-    def impl(*args, **kwargs):
-        raise RuntimeError(f"xgen_amd.{name}: native operators not found at {path}; build them with "
-                           "`python -c 'import __graft_entry__ as g; g.build()'`")
+_LOAD_LOCK = threading.Lock()
+_native_loaded = False
+
+
+def _load_native() -> None:
+    """Loads the native operators' library, which registers them under the CUDA key, unless it is loaded.
+    RuntimeError if it is absent or does not load: there is no other implementation of these operators."""
+    global _native_loaded
+    with _LOAD_LOCK:
+        if _native_loaded:
+            return
+        path, build = N.operators_path(), "build them with `python -c 'import __graft_entry__ as g; g.build()'`"
+        if not path.is_file():
+            raise RuntimeError(f"xgen_amd native operators not found at {path}; {build}")
+        try:
+            torch.ops.load_library(str(path))
+        except OSError as error:
+            raise RuntimeError(f"xgen_amd native operators at {path} do not load ({error}); {build}") from error
+        _native_loaded = True
+
+
+def _stand_in(name: str):
+    """The operator while its native implementation is not there: a call loads the library, built since, or
+    says why it cannot.  Registered below every backend's own kernel, so that the loaded one takes over."""
+    def impl(*args):
+        _load_native()
+        device = args[0].device
+        if device.type != "cuda":
+            raise NotImplementedError(f"Could not run '{NAMESPACE}::{name}' with arguments from the "
+                                      f"'{device.type.upper()}' backend")
+        return getattr(xops, name)(*args)
     return impl
 
 
 def register() -> None:
-    """Defines the xgen_amd operators (idempotent; does not load the HIP library)."""
+    """Defines the xgen_amd operators (idempotent; does not load the HIP library).  A native operators'
+    library that is absent or does not load is left to the first call."""
     global _LIB
     if _LIB is not None:
         return
@@ -294,13 +324,12 @@ def register() -> None:
         lib.define(schema)
         lib.impl(name, _META[name], "Meta")
     lib.impl("swiglu_quant", _swiglu_gpu, "CUDA")
-    path = N.operators_path()
-    if path.is_file():
-        torch.ops.load_library(str(path))
-    else:  # no other implementation of these operators exists: calls say so
+    try:
+        _load_native()
+    except RuntimeError:
         for name in _META:
             if name != "swiglu_quant":
-                lib.impl(name, _not_built(name, path), "CUDA")
+                lib.impl(name, _stand_in(name), "CompositeExplicitAutograd")
     _LIB = lib
 
 
