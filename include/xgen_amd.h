@@ -27,6 +27,8 @@
 extern "C" {
 #endif
 
+/* raised when an entry point changes or goes; a library from before one was added has the same
+ * version and lacks the symbol (since version 1: xgen_fp8_quantize_tensor) */
 #define XGEN_ABI_VERSION 1
 
 /* status codes */

@@ -23,6 +23,15 @@ def built_library():
     return path
 
 
+def library_without(library, symbol: str, folder):
+    """A copy of libxgen_amd.so that does not export `symbol`: what an older build of the same ABI version is."""
+    data, name = library.read_bytes(), b"\0" + symbol.encode() + b"\0"
+    assert name in data
+    copy = folder / "older.so"
+    copy.write_bytes(data.replace(name, name[:-2] + b"_\0"))
+    return copy
+
+
 @pytest.fixture(scope="session")
 def cuda():
     import torch

@@ -2,10 +2,14 @@
 library and declared to ctypes; argument validation fails before any HIP call
 (no GPU needed)."""
 import ctypes
+import os
 import re
+import subprocess
+import sys
 
 import pytest
 
+from conftest import library_without
 from xgen_amd import _native as N
 
 HEADER = N.Path(__file__).resolve().parents[1] / "include" / "xgen_amd.h"
@@ -38,6 +42,28 @@ def test_status_strings(built_library):
     assert L.xgen_abi_version() == 1
     assert L.xgen_status_string(N.OK) == b"ok"
     assert L.xgen_status_string(N.ERR_UNSUPPORTED) == b"unsupported shape or layout"
+
+
+LOAD = r"""
+import sys
+sys.path.insert(0, sys.argv[1])
+from xgen_amd import _native as N
+try:
+    print(N.lib().xgen_abi_version())
+except Exception as error:
+    print(type(error).__name__, error)
+"""
+
+
+@pytest.mark.parametrize("symbol,says", [("xgen_fp8_quantize_tensor", "1"),
+                                         ("xgen_merge_quant", "RuntimeError {path}: undefined symbol: xgen_merge_quant")])
+def test_library_without_a_symbol(built_library, tmp_path, symbol, says):
+    """A library of this ABI version from before an entry point was added to it still loads; one without any
+    other is refused with its path and the symbol."""
+    older = library_without(built_library, symbol, tmp_path)
+    proc = subprocess.run([sys.executable, "-c", LOAD, str(HEADER.parents[1])], stdout=subprocess.PIPE,
+                          stderr=subprocess.STDOUT, text=True, timeout=120, env={**os.environ, "XGEN_AMD_LIBRARY": str(older)})
+    assert proc.stdout.strip().splitlines()[-1] == says.format(path=older)
 
 
 _STRIDES = (N._c_i64 * 12)(384, 128, 128, 128, 384, 128, 128, 128, 384, 128, 128, 128)

@@ -1,5 +1,9 @@
 """GPU parity of the quantizers: bytes and scales bit-exact against the oracle."""
 import math
+import os
+import subprocess
+import sys
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -7,6 +11,7 @@ import torch
 
 import oracle.ref as R
 import xgen_amd  # noqa: F401
+from conftest import library_without
 from xgen_amd import _native as N
 from xgen_amd import workloads
 from xgen_amd.operator.h3_abs_peak import activation_abs_peak
@@ -144,6 +149,32 @@ def test_quantize_tensor_equals_scale_then_pack(cuda, dtype, numel):
         want = xops.fp8_tensor_scale(v)
         assert torch.equal(scale.view(torch.int32), want.view(torch.int32))
         assert torch.equal(q.view(torch.uint8), xops.fp8_pack(v, want).view(torch.uint8))
+
+
+OLDER = r"""
+import sys
+sys.path.insert(0, sys.argv[1])
+import torch
+from xgen_amd.operator.h3_fp8_quant import quantize_activation
+x = torch.load(sys.argv[2], weights_only=True).cuda()
+q, scale = quantize_activation(x)
+rows = torch.ops.xgen_amd.quantize_rows(x, torch.int8)[0]
+torch.save((q.view(torch.uint8).cpu(), scale.cpu(), rows.cpu()), sys.argv[3])
+"""
+
+
+def test_library_from_before_quantize_tensor(cuda, tmp_path):
+    """XGEN_AMD_LIBRARY names a library of this ABI version without xgen_fp8_quantize_tensor: the operators
+    run on it, the per-tensor quantization in its two calls."""
+    older = library_without(N.library_path(), "xgen_fp8_quantize_tensor", tmp_path)
+    x = torch.randn((37, 264), generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    torch.save(x, tmp_path / "x.pt")
+    subprocess.run([sys.executable, "-c", OLDER, str(Path(__file__).resolve().parents[1]), str(tmp_path / "x.pt"),
+                    str(tmp_path / "out.pt")], check=True, timeout=100, env={**os.environ, "XGEN_AMD_LIBRARY": str(older)})
+    q, scale, rows = torch.load(tmp_path / "out.pt", weights_only=True)
+    want, want_scale = xops.fp8_quantize_tensor(x.to(cuda))
+    assert torch.equal(q, want.view(torch.uint8).cpu()) and torch.equal(scale, want_scale.cpu())
+    assert torch.equal(rows, xops.quantize_rows(x.to(cuda), torch.int8)[0].cpu())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

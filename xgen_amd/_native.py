@@ -101,6 +101,10 @@ SIGNATURES = {
 }
 
 
+# added within ABI version 1: a library from before them still loads
+ADDED = frozenset({"xgen_fp8_quantize_tensor"})
+
+
 def library_path() -> Path:
     default = Path(__file__).resolve().parent / "_lib" / "libxgen_amd.so"
     return Path(os.environ.get("XGEN_AMD_LIBRARY", default)).resolve()
@@ -125,7 +129,11 @@ def lib() -> ctypes.CDLL:
                     "`python -c 'import __graft_entry__ as g; g.build()'`")
             handle = ctypes.CDLL(str(path))
             for name, (restype, argtypes) in SIGNATURES.items():
-                fn = getattr(handle, name)
+                fn = getattr(handle, name, None)
+                if fn is None:
+                    if name in ADDED:
+                        continue
+                    raise RuntimeError(f"{path}: undefined symbol: {name}")
                 fn.restype = restype
                 fn.argtypes = argtypes
             if handle.xgen_abi_version() != 1:

@@ -29,11 +29,12 @@ struct Api {
 #define XGEN_API(X)                                                                                         \
   X(xgen_status_string) X(xgen_last_error) X(xgen_quantize_rows) X(xgen_quantize_rows_gelu)                 \
   X(xgen_abs_peak_workspace_bytes) X(xgen_abs_peak) X(xgen_fp8_tensor_scale) X(xgen_fp8_pack)               \
-  X(xgen_fp8_quantize_tensor)                                                                               \
   X(xgen_norm_affine_quant) X(xgen_scaled_mm_fp8) X(xgen_scaled_mm_fp8_exact) X(xgen_quant_matmul_int8)     \
   X(xgen_gate_residual) X(xgen_indexed_modulate) X(xgen_merge_quant) X(xgen_w8a8_gate_residual)
 #define XGEN_FIELD(f) decltype(&::f) f;
   XGEN_API(XGEN_FIELD)
+  // added within ABI version 1: null where XGEN_AMD_LIBRARY names a library from before it
+  decltype(&::xgen_fp8_quantize_tensor) xgen_fp8_quantize_tensor;
 };
 
 Api open_api() {
@@ -57,6 +58,8 @@ Api open_api() {
   a.f = reinterpret_cast<decltype(&::f)>(dlsym(handle, #f));              \
   TORCH_CHECK(a.f, path, ": undefined symbol ", #f);
   XGEN_API(XGEN_RESOLVE)
+  a.xgen_fp8_quantize_tensor =
+      reinterpret_cast<decltype(&::xgen_fp8_quantize_tensor)>(dlsym(handle, "xgen_fp8_quantize_tensor"));
   const auto version = reinterpret_cast<decltype(&::xgen_abi_version)>(dlsym(handle, "xgen_abi_version"));
   TORCH_CHECK(version && version() == XGEN_ABI_VERSION, path, ": unexpected ABI version");
   return a;
@@ -188,6 +191,10 @@ std::tuple<Tensor, Tensor> fp8_quantize_tensor(const Tensor &x) {
   on_gpu(x);
   TORCH_CHECK(is_half(x), "abs_peak: BF16/F16 input required");
   TORCH_CHECK(x.numel() > 0, "xgen_fp8_tensor_scale: empty input");
+  if (!api().xgen_fp8_quantize_tensor) {  // the same scale and bytes in two calls
+    const Tensor scale = fp8_tensor_scale(x);
+    return {fp8_pack(x, scale), scale};
+  }
   const c10::DeviceGuard guard(x.device());
   Tensor q = empty(x.sizes(), at::kFloat8_e4m3fn, x), scale = empty({}, at::kFloat, x);
   const Tensor xc = aligned_flat(x);
