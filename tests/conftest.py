@@ -23,6 +23,21 @@ def built_library():
     return path
 
 
+GEMM_KINDS = {"int8": 0, "fp8": 1, "fp8_exact": 2}
+
+
+def gemm_tile(kind: str, M: int, Nf: int, K: int, gated: bool = False, accumulators: bool = False):
+    """(rows, columns) of the output tiles that such a W8A8 GEMM call runs on, asked of the library."""
+    import ctypes
+    from xgen_amd import _native
+    fn = ctypes.CDLL(str(_native.library_path())).xgen_gemm_tile_choice
+    fn.restype = ctypes.c_int
+    fn.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3 + [ctypes.c_int] * 2 + [ctypes.POINTER(ctypes.c_int)]
+    n = ctypes.c_int()
+    m = fn(GEMM_KINDS[kind], M, Nf, K, int(gated), int(accumulators), ctypes.byref(n))
+    return m, n.value
+
+
 def library_without(library, symbol: str, folder):
     """A copy of libxgen_amd.so that does not export `symbol`: what an older build of the same ABI version is."""
     data, name = library.read_bytes(), b"\0" + symbol.encode() + b"\0"
