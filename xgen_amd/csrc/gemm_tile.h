@@ -17,9 +17,10 @@
 // so a pair's DMA has SLOTS - 1 pairs of work in front of it.
 //
 // What bounds it: a tile's K steps are a serial chain, so a few hundred tokens
-// cost K / 128 steps of ~0.15 us whatever the number of workgroups below the
-// CUs' (256 x 1,024 x 1,024: 14.1 us on 256 x 256 tiles, 4 of them; 4.0 us on 128
-// tiles of 32 x 64).  From about one 128 x 192 tile per CU on it is the board's
+// cost K / 128 steps whatever the number of workgroups below the CUs'.  On 32 x 64
+// with the weights in the last-level cache a step takes 0.16 us, 0.34 in the exact
+// kind (from memory: kTileCosts); 256 x 1,024 x 1,024 so takes 4.7 us on 128 such
+// tiles, 15 on 4 tiles of 256 x 256 (exact kind 6.2 and 24).  From about one 128 x 192 tile per CU on it is the board's
 // power: M = 1,955, N = 3,072, K = 12,288 on 256 tiles takes 62 us (2.37 PFLOP/s;
 // 104 us on 96 tiles of 256 x 256), 49 us with all operands zero, and 59 us with
 // the fragment reads taken out.  Per flop a smaller tile moves more data through

@@ -226,7 +226,9 @@ struct MfmaA<kFp8Exact> {
   static __device__ __forceinline__ void mma0(f32x16 &c, const i32x8 &w, const xw_t &xb) { run<true>(c, w, xb); }
   static __device__ __forceinline__ void mma(f32x16 &c, const i32x8 &w, const i32x8 &x) { run<false>(c, w, widen_x(x)); }
   static __device__ __forceinline__ void mma0(f32x16 &c, const i32x8 &w, const i32x8 &x) { run<true>(c, w, widen_x(x)); }
-};// 128-byte rows: 16-byte chunk c of row r at c ^ ((r >> 1) & 7); the 16 lanes of
+};
+
+// 128-byte rows: 16-byte chunk c of row r at c ^ ((r >> 1) & 7); the 16 lanes of
 // one 128-bit access (rows r..r+15, one chunk) hit 16 distinct bank groups.
 __device__ __forceinline__ int swz128(int row, int chunk) { return row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4); }
 template <int KIND>

@@ -648,8 +648,8 @@ int gemm_entry(const char *fn, const void *a, int64_t lda, const void *w, int64_
   }
   // The kernels address the activation rows, the output rows and the residual rows through 32-bit
   // buffer offsets (rows past M of the last tile-row included).  A call whose rows pass those
-  // limits runs as consecutive launches over row chunks: each output row is computed by the same
-  // tiles in the same K order whichever launch it falls in, so the results are those of one launch.
+  // limits runs as consecutive launches over row chunks: an output's products are summed in the same
+  // order whichever launch and tile it falls in, so the results are those of one launch.
   int64_t rows = M;
   auto cap = [&](int64_t limit) { rows = limit < rows ? limit : rows; };
   cap((0x7fffffffLL - K) / lda + 1);                   // activation bytes below 2^31

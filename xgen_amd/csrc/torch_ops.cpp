@@ -1,8 +1,8 @@
 // CUDA-key implementations of the xgen_amd operators (xgen_amd/ops.py defines their schemas and
 // Meta implementations): argument checks, outputs from the caching allocator, one C ABI call on
-// the tensors' current stream.  Native because a small call is bound by this work: from Python
-// an operator cost ~17 us of host time (a 256 x 1,024 x 1,024 projection, two operators and 8 us
-// of kernels, 35 us a call); from here ~5 us.
+// the tensors' current stream.  Native because a small call is bound by this work: in Python
+// an operator took 13 to 15 us of host time with its launch (a 256 x 1,024 x 1,024 projection, two
+// operators and 8 us of kernels under a module, 35 us a call); from here 5 to 6 (17 us a call).
 //
 // This library links torch only.  The kernels' library is opened on the first operator call, from
 // XGEN_AMD_LIBRARY or this library's own folder, as xgen_amd/_native.py opens it.
