@@ -18,8 +18,9 @@ def built_library():
     from xgen_amd import _native
     path = _native.library_path()
     if not (path.is_file() and _native.operators_path().is_file()):
-        from xgen_amd import _build
+        from xgen_amd import _build, ops
         _build.build()
+        ops._load_native()
     return path
 
 

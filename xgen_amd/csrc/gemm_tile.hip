@@ -54,9 +54,10 @@ constexpr TileCost kTileCosts[3][kTiles + 1] = {
 // The 256 x 256 kernel keeps a call unless a smaller tile is put 4% below it.  On short K, where
 // the sums put its epilogue too high, 10%: up to K = 512, and against the tiles from 128 x 192 on up
 // to 1,024 (at 4%, 1,955 x 18,432 x 64 exact: 37.6 us on 256 x 192, 31.6 there).  So 35 of 5,748
-// calls on those shapes are more than 3% slower than on it, 9% at most.  A gated call's epilogue is what a smaller tile saves most: 4% for all of them, and of 840
-// none is slower (3,906 x 3,072 x 3,072 FP8: 40.6 against 45.8 us).  A call that stores its
-// accumulators stores three times the bytes, on the 256-row tiles all at the end: 15% for them (at
+// calls on those shapes are more than 3% slower than on it, 14% at most (15,624 x 5,376 x 320 exact,
+// 7% in another run).  A gated call's epilogue is what a smaller tile saves most: 4% for all of
+// them, and of 1,894 none is slower (3,906 x 3,072 x 3,072 FP8: 40.6 against 45.8 us).  A call that
+// stores its accumulators stores three times the bytes, on the 256-row tiles all at the end: 15% for them (at
 // the lines above, 15,624 x 5,376 x 384 exact: 228 us on 256 x 192, 148 on the large kernel, and 44
 // of 1,776 calls more than 3% slower than on it; so 18, most of them under K = 1,024, 17% at most).
 float keep_large(int tile, int64_t K, bool gated, bool accumulators) {
